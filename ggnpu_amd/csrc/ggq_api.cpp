@@ -47,6 +47,18 @@ struct Work {
     Buffer part;  // GEMM split-K partial tiles
 };
 
+// Planes of the activation rows of the fp16 GEMM, one buffer per stream: the
+// calls that take that GEMM also run at sizes and activation treatments that
+// need no other workspace, and callers may queue those on several streams at
+// once.  At most kMaxLanes streams of a context have one; calls on further
+// streams take the kernels that need none.
+struct Lane {
+    hipStream_t stream = nullptr;
+    Buffer b;
+    unsigned long long capture = 0;  // the capture whose graph holds the buffer's address (0: none)
+};
+constexpr size_t kMaxLanes = 8, kMaxCapturedLanes = 16;
+
 }  // namespace
 
 struct ggq_ctx {
@@ -60,6 +72,8 @@ struct ggq_ctx {
     Work dev;   // workspace of the *_dev entry points
     Work host;  // workspace of the synchronous host-pointer entry points (never
                 // shared with device calls that may still run on other streams)
+    std::vector<Lane> lanes;     // workspace of the fp16 GEMM on the *_dev entry points
+    size_t captured_lanes = 0;   // lane buffers that captured graphs keep
     Buffer io;  // staging of host A / C for the synchronous entry points
     Buffer logits;  // vocab projection output when the caller does not keep it
     Buffer attn;  // attention chunk partials
@@ -119,6 +133,58 @@ int grow(ggq_ctx* c, Buffer& b, size_t need, hipStream_t s, const char* what) {
     return GGQ_OK;
 }
 
+// `bytes` of the stream's lane, or null when it cannot have them now (the
+// caller then takes a path without this workspace): more streams than lanes,
+// no memory, hipStreamPerThread (one handle for several streams), or a
+// capture that would have to allocate.  A buffer that a captured graph uses
+// is left to that graph: later calls on the stream get another one, so a
+// replay on some other stream never meets them.
+void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
+    if (s == hipStreamPerThread) return nullptr;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(s, &cs, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    Lane* l = nullptr;
+    for (Lane& x : c->lanes)
+        if (x.stream == s) l = &x;
+    if (cs != hipStreamCaptureStatusNone) {
+        if (cs != hipStreamCaptureStatusActive || !l || l->b.size < bytes) return nullptr;
+        if (l->capture != id) {
+            if (l->capture || c->captured_lanes >= kMaxCapturedLanes) return nullptr;
+            l->capture = id;
+            c->captured_lanes++;
+        }
+        return l->b.ptr;
+    }
+    if (!l) {
+        if (c->lanes.size() >= kMaxLanes) return nullptr;
+        c->lanes.emplace_back();
+        l = &c->lanes.back();
+        l->stream = s;
+    }
+    if (l->capture || l->b.size < bytes) {
+        // relaxed: the allocation is no part of a capture another thread may
+        // have running
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        hipThreadExchangeStreamCaptureMode(&mode);
+        void* p = nullptr;
+        const size_t sz = l->capture ? std::max(bytes, l->b.size) : std::max(bytes, 2 * l->b.size);
+        const hipError_t e = hipMalloc(&p, sz);
+        hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (l->b.ptr) c->retired.push_back(l->b.ptr);
+        l->b = Buffer{p, sz};
+        l->capture = 0;
+    }
+    return l->b.ptr;
+}
+
 inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Where a call's scratch memory comes from: the growable buffers of a Work,
@@ -149,6 +215,14 @@ struct Arena {
         *part = part_bytes ? (float*)(fixed + off) : nullptr;
         return GGQ_OK;
     }
+    // Planes of the fp16 GEMM beside `ws_bytes` taken with get(), or null
+    // when the call should run without them.
+    void* planes(size_t ws_bytes, size_t bytes) {
+        if (w == &c->dev) return lane_ws(c, s, bytes);
+        if (w) return grow(c, w->part, bytes, s, "workspace") == GGQ_OK ? w->part.ptr : nullptr;
+        const size_t off = align256(ws_bytes);
+        return off + bytes <= cap ? fixed + off : nullptr;
+    }
 };
 
 Arena dev_arena(ggq_ctx* c, hipStream_t s) { return Arena{c, &c->dev, nullptr, 0, s}; }
@@ -176,6 +250,81 @@ int check_matmul_shape(ggq_ctx* c, uint32_t type, int64_t N, int64_t K, int M, i
     return GGQ_OK;
 }
 
+// The matmuls that run on the fp16 GEMM: one activation matrix (fp32 rows A,
+// as they are or quantized per row, or int8 codes qa with row scales sa) and
+// the weights that share it.
+struct GemmEntry {
+    const void* W;
+    uint32_t type;
+    int N;
+    float* C;
+    int ldc;
+};
+constexpr int kGemmMinRows = 9;
+enum { GEMM_F32 = 0, GEMM_Q8_ROW = 1, GEMM_CODES = 2 };
+
+// Q8_0 and IQ4_NL rows of codes stay on the int8 GEMMs, whose 32-value dots
+// are exact: their weights would take two planes here.
+bool gemm_f16_takes(uint32_t type, int M, int mode) {
+    return M >= kGemmMinRows && (mode == GEMM_F32 || (type != GGQ_TYPE_Q8_0 && type != GGQ_TYPE_IQ4_NL));
+}
+
+// Rows per pass over the weights: the planes of a pass stay within 256 MB.
+int gemm_rows_per_pass(int K, int M, bool codes) {
+    const size_t row = ggq::gemm_f16_ws_bytes(K, 64, codes) / 64;
+    const size_t rows = ((size_t(256) << 20) / row) & ~size_t(63);
+    return (size_t)M <= rows ? M : (int)std::max<size_t>(rows, 64);
+}
+
+// True when the call was taken (*st its status); false: not queued.
+bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n, int K, int mode, const float* A,
+              int lda, const int8_t* qa, const float* sa, int M, hipStream_t s, int* st) {
+    const bool codes = mode != GEMM_F32;
+    const int step = gemm_rows_per_pass(K, M, codes);
+    void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
+    if (!ws) return false;
+    hipError_t e;
+    for (int m0 = 0; m0 < M; m0 += step) {
+        const int rows = std::min(step, M - m0);
+        e = ggq::launch_gemm_f16_prep(mode, A ? A + (size_t)m0 * lda : nullptr, lda, qa ? qa + (size_t)m0 * K : nullptr,
+                                      K, rows, ws, s);
+        if (e != hipSuccess) return *st = hip_status(c, e, "gemm_f16 rows"), true;
+        bool done[GGQ_MAX_BATCH] = {};
+        for (int i = 0; i < n; i++) {
+            if (done[i]) continue;
+            ggq::GemmDesc gd[GGQ_MAX_GEMM_BATCH];
+            int ng = 0;
+            for (int j = i; j < n && ng < GGQ_MAX_GEMM_BATCH; j++)
+                if (!done[j] && d[j].type == d[i].type) {
+                    gd[ng++] = ggq::GemmDesc{d[j].W, d[j].C + (size_t)m0 * d[j].ldc, d[j].N, d[j].ldc};
+                    done[j] = true;
+                }
+            e = ggq::launch_gemm_f16(d[i].type, gd, ng, K, rows, codes, sa ? sa + m0 : nullptr, ws, s);
+            if (e != hipSuccess) return *st = hip_status(c, e, "gemm_f16"), true;
+        }
+    }
+    return *st = set_status(c, GGQ_OK), true;
+}
+
+// The entries of a batch on the fp16 GEMM, those that share their activations
+// and K together; done[i] marks the entries queued.
+int gemm_f16_shared(ggq_ctx* c, Arena& ar, const ggq_gemv_desc* d, int n, int M, int mode, hipStream_t s, bool* done) {
+    for (int i = 0; i < n; i++) {
+        if (done[i] || !gemm_f16_takes(d[i].type, M, mode)) continue;
+        GemmEntry ge[GGQ_MAX_BATCH];
+        int idx[GGQ_MAX_BATCH], ng = 0, st;
+        for (int j = i; j < n; j++)
+            if (!done[j] && d[j].A == d[i].A && d[j].K == d[i].K && gemm_f16_takes(d[j].type, M, mode)) {
+                idx[ng] = j;
+                ge[ng++] = GemmEntry{d[j].W, d[j].type, (int)d[j].N, d[j].C, (int)d[j].N};
+            }
+        if (!gemm_f16(c, ar, 0, ge, ng, (int)d[i].K, mode, d[i].A, (int)d[i].K, nullptr, nullptr, M, s, &st)) continue;
+        if (st != GGQ_OK) return st;
+        for (int j = 0; j < ng; j++) done[idx[j]] = true;
+    }
+    return GGQ_OK;
+}
+
 // Queues C = A . W^T with the requested activation treatment.
 int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N, int64_t K, const float* A,
                   int lda, float* C, int ldc, int M, int act_mode, hipStream_t s) {
@@ -191,7 +340,9 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     g.ldy = ldc;
     g.M = M;
     g.groups = 1;
+    const GemmEntry ge{W, type, (int)N, C, ldc};
     if (act_mode == GGQ_ACT_F32) {
+        if (gemm_f16_takes(type, M, GEMM_F32) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_F32, A, lda, nullptr, nullptr, M, s, &st)) return st;
         g.X = A;
         g.ldx = lda;
         return hip_status(c, ggq::launch_gemv(g, s), "gemv");
@@ -209,6 +360,9 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
         if (ggq::i8_gemv_eligible(&g, 1, 1))
             return hip_status(c, ggq::launch_i8_gemv(&g, 1, 1, nullptr, nullptr, s), "gemv_i8");
     }
+    if (act_mode == GGQ_ACT_Q8_ROW && gemm_f16_takes(type, M, GEMM_Q8_ROW) &&
+        gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_Q8_ROW, A, lda, nullptr, nullptr, M, s, &st))
+        return st;
     if (act_mode == GGQ_ACT_Q8_ROW && M > 8 && ggq::gemm_panel_eligible(type, (int)K, M, A, lda)) {
         // quantized per row inside the GEMM (no workspace)
         const ggq::GemmDesc gd{W, C, (int)N, ldc};
@@ -234,6 +388,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     }
     if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, nullptr, nullptr, xe, s)) != hipSuccess)
         return hip_status(c, e, "quant_act");
+    if (gemm_f16_takes(type, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
     g.X = xe;
     g.ldx = (int)K;
     return hip_status(c, ggq::launch_gemv(g, s), "gemv");
@@ -247,6 +402,8 @@ int mul_mat_q8_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_
     int st;
     void* ws;
     float* part;
+    const GemmEntry ge{W, type, (int)N, C, ldc};
+    if (gemm_f16_takes(type, M, GEMM_CODES) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_CODES, nullptr, 0, qa, sa, M, s, &st)) return st;
     if (M > 8 && ggq::gemm_panel_eligible(type, (int)K, M, nullptr, 0)) {
         const ggq::GemmDesc gd{W, C, (int)N, ldc};
         return hip_status(c, ggq::launch_gemm_panel(type, &gd, 1, (int)K, nullptr, 0, qa, sa, M, s), "gemm_panel");
@@ -433,6 +590,8 @@ void ggq_destroy(ggq_ctx* c) {
     for (Buffer* b : {&c->dev.ws, &c->dev.part, &c->host.ws, &c->host.part})
         if (b->ptr) hipFree(b->ptr);
     for (void* p : c->retired) hipFree(p);
+    for (Lane& l : c->lanes)
+        if (l.b.ptr) hipFree(l.b.ptr);
     if (c->io.ptr) hipFree(c->io.ptr);
     if (c->logits.ptr) hipFree(c->logits.ptr);
     if (c->attn.ptr) hipFree(c->attn.ptr);
@@ -652,6 +811,12 @@ int ggq_mul_mat_q8_batch_dev(ggq_ctx* c, const ggq_gemm_desc* d, int n, uint32_t
     if (M == 0) return set_status(c, GGQ_OK);
     const hipStream_t s = pick_stream(c, stream);
     Arena ar = dev_arena(c, s);
+    if (gemm_f16_takes(type, M, GEMM_CODES)) {
+        GemmEntry ge[GGQ_MAX_GEMM_BATCH];
+        for (int i = 0; i < n; i++) ge[i] = GemmEntry{d[i].W, type, (int)d[i].N, d[i].C, d[i].ldc};
+        int st;
+        if (gemm_f16(c, ar, 0, ge, n, (int)K, GEMM_CODES, nullptr, 0, qa, sa, M, s, &st)) return st;
+    }
     if (M <= 8 || type == GGQ_TYPE_Q6_K) {
         for (int i = 0; i < n; i++) {
             const int st = mul_mat_q8_queue(c, ar, d[i].W, type, d[i].N, K, qa, sa, M, d[i].C, d[i].ldc, s);
@@ -698,7 +863,18 @@ int ggq_mul_mat_batch_rows_dev(ggq_ctx* c, const ggq_gemv_desc* d, int n, int M,
         ps[i].groups = 1;
     }
     if (M == 0) return set_status(c, GGQ_OK);
-    return hip_status(c, ggq::launch_gemv_multi(ps, n, pick_stream(c, stream)), "gemv batch");
+    const hipStream_t s = pick_stream(c, stream);
+    bool done[GGQ_MAX_BATCH] = {};
+    if (M >= kGemmMinRows) {
+        Arena ar = dev_arena(c, s);
+        const int st = gemm_f16_shared(c, ar, d, n, M, GEMM_F32, s, done);
+        if (st != GGQ_OK) return st;
+    }
+    int left = 0;
+    for (int i = 0; i < n; i++)
+        if (!done[i]) ps[left++] = ps[i];
+    if (!left) return set_status(c, GGQ_OK);
+    return hip_status(c, ggq::launch_gemv_multi(ps, left, s), "gemv batch");
     GGQ_END(c)
 }
 
@@ -782,6 +958,11 @@ int ggq_mul_mat_batch_act_dev(ggq_ctx* c, const ggq_gemv_desc* d, int n, int M, 
     if (act_mode == GGQ_ACT_Q8_ROW && M <= 8 && ggq::i8_gemv_eligible(ps, n, 1))
         return hip_status(c, ggq::launch_i8_gemv(ps, n, 1, nullptr, nullptr, s), "gemv_i8 batch");
     bool done[GGQ_MAX_BATCH] = {};
+    if (act_mode == GGQ_ACT_Q8_ROW && M >= kGemmMinRows) {
+        Arena ar = dev_arena(c, s);
+        const int st = gemm_f16_shared(c, ar, d, n, M, GEMM_Q8_ROW, s, done);
+        if (st != GGQ_OK) return st;
+    }
     if (act_mode == GGQ_ACT_Q8_ROW && M > 8) {
         // Prefill-sized: entries that share the activations, type and K (q/k/v,
         // gate/up) as one activation-panel GEMM that quantizes the rows itself.

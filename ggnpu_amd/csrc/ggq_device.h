@@ -538,6 +538,14 @@ __device__ __forceinline__ void ubytes_to_f32(uint4 u, float* f) {
     }
 }
 
+// int8 code of an activation divided by its scale: clamp(nearbyint(v), -128,
+// 127) (amd_xdna.cpp:598-603, 757-771); rint is IEEE half-to-even.
+__device__ __forceinline__ int8_t to_i8(float v) {
+    float r = __builtin_rintf(v);
+    r = fminf(fmaxf(r, -128.0f), 127.0f);
+    return (int8_t)(int)r;
+}
+
 // ------------------------------------------------- MoE chunk lists -----
 // (group, first row) chunk lists for grouped launches (struct ChunkList,
 // ggq_launch.h).

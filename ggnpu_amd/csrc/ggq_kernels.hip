@@ -119,13 +119,7 @@ hipError_t launch_block_dot(uint32_t type, const void* W, int N, int K, const in
 
 // ========================================================= activation quant
 // Reference: amd_xdna.cpp:633-639 (scale = amax/127, or 1 for a zero row) and
-// :598-603, :757-771 (q = clamp(nearbyint(a * (1/scale)), -128, 127)).
-// Division and rint are IEEE (correctly rounded / half-to-even).
-__device__ __forceinline__ int8_t to_i8(float v) {
-    float r = __builtin_rintf(v);
-    r = fminf(fmaxf(r, -128.0f), 127.0f);
-    return (int8_t)(int)r;
-}
+// :598-603, :757-771; the codes are to_i8 (ggq_device.h) of a * (1/scale).
 
 // Sum over the 256 threads of a workgroup (four wavefronts), in a fixed
 // order; every thread gets the total.

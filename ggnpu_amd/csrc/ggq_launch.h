@@ -146,6 +146,18 @@ hipError_t launch_gemm_i8(uint32_t type, const void* W, int N, int K, const int8
 bool gemm_panel_eligible(uint32_t type, int K, int M, const float* A, int lda);
 hipError_t launch_gemm_panel(uint32_t type, const GemmDesc* d, int n, int K, const float* A, int lda,
                              const int8_t* qa, const float* sa, int M, hipStream_t s);
+// GEMM on fp16 planes of the activation rows (ggq_gemm_f16.hip), every type
+// and K.  launch_gemm_f16_prep writes the planes of M rows into `ws`
+// (gemm_f16_ws_bytes, 256-byte aligned; codes: one plane, else two): mode 0
+// fp32 rows A [M][lda], 1 the same quantized per row (codes and scales of
+// launch_quant_act mode 1), 2 given int8 codes qa [M][K] (8-byte aligned,
+// row scales `sa` passed to launch_gemm_f16).  launch_gemm_f16 multiplies
+// them with up to 4 weights of one type.
+size_t gemm_f16_ws_bytes(int K, int M, bool codes);
+hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t* qa, int K, int M, void* ws,
+                                hipStream_t s);
+hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, bool codes, const float* sa,
+                           const void* ws, hipStream_t s);
 // idx[m] = first index of the largest value of row m of L ([M][ld], N
 // values); val[m] = that value (val may be null).  `ws`: device workspace
 // of argmax_workspace_bytes(M) bytes.
