@@ -263,17 +263,37 @@ struct GemmEntry {
 constexpr int kGemmMinRows = 9;
 enum { GEMM_F32 = 0, GEMM_Q8_ROW = 1, GEMM_CODES = 2 };
 
-// Q8_0 and IQ4_NL rows of codes stay on the int8 GEMMs, whose 32-value dots
-// are exact: their weights would take two planes here.
-bool gemm_f16_takes(uint32_t type, int M, int mode) {
-    return M >= kGemmMinRows && (mode == GEMM_F32 || (type != GGQ_TYPE_Q8_0 && type != GGQ_TYPE_IQ4_NL));
+// Whether M rows against `cols` columns of one type run on the fp16 GEMM
+// (times in us, earlier kernels -> fp16 GEMM).
+//   fp32 rows: the decode GEMVs' passes of four rows are cheaper for small
+//   weights (1024 x 1024 Q4_K, 64 rows: 7.6 -> 10.6; 2048 x 2048 Q6_K, 16
+//   rows: 10.1 -> 10.7, 32 rows: 13.7 -> 12.3; 512 x 2048, 200 rows: 16.7 ->
+//   18.4, 500 rows: 28.9 -> 22.4); Q8_0 and IQ4_NL blocks load as 8 scales
+//   and 8 runs and win later (2048 x 2048 Q8_0, 32 rows: 14.3 -> 18.7, 64 rows:
+//   20.4 -> 20.1).
+//   int8 codes: Q8_0 and IQ4_NL stay on the int8 GEMMs, which take the blocks'
+//   codes as they are (two planes here: 512 x 1536 rows 131 -> 243 a layer);
+//   so does IQ4_XS above the activation panel's K (2048 x 8192, 32 / 500 rows:
+//   18 -> 22, 47 -> 57) and Q4_K / Q5_K there up to 64 rows (20.7 -> 23.7).
+bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
+    if (M < kGemmMinRows) return false;
+    const bool blocks32 = type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL;
+    const int64_t w = cols * K, work = w * M;
+    if (mode == GEMM_F32) {
+        if (blocks32) return M >= 48 && work >= (int64_t)256 << 20;
+        return work >= (w >= 1 << 22 ? (int64_t)80 << 20 : (int64_t)256 << 20);
+    }
+    if (type == GGQ_TYPE_Q6_K) return true;
+    if (blocks32) return false;
+    if (K <= 2048) return true;
+    return type != GGQ_TYPE_IQ4_XS && (M <= 32 || M > 64);
 }
 
 // Rows per pass over the weights: the planes of a pass stay within 256 MB.
 int gemm_rows_per_pass(int K, int M, bool codes) {
-    const size_t row = ggq::gemm_f16_ws_bytes(K, 64, codes) / 64;
-    const size_t rows = ((size_t(256) << 20) / row) & ~size_t(63);
-    return (size_t)M <= rows ? M : (int)std::max<size_t>(rows, 64);
+    const size_t row = ggq::gemm_f16_ws_bytes(K, 128, codes) / 128;
+    const size_t rows = ((size_t(256) << 20) / row) & ~size_t(127);
+    return (size_t)M <= rows ? M : (int)std::max<size_t>(rows, 128);
 }
 
 // True when the call was taken (*st its status); false: not queued.
@@ -309,16 +329,22 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
 // The entries of a batch on the fp16 GEMM, those that share their activations
 // and K together; done[i] marks the entries queued.
 int gemm_f16_shared(ggq_ctx* c, Arena& ar, const ggq_gemv_desc* d, int n, int M, int mode, hipStream_t s, bool* done) {
+    bool seen[GGQ_MAX_BATCH] = {};
     for (int i = 0; i < n; i++) {
-        if (done[i] || !gemm_f16_takes(d[i].type, M, mode)) continue;
+        if (seen[i]) continue;
+        int64_t cols = 0;
+        for (int j = i; j < n; j++)
+            if (d[j].A == d[i].A && d[j].K == d[i].K) cols += d[j].N;
         GemmEntry ge[GGQ_MAX_BATCH];
         int idx[GGQ_MAX_BATCH], ng = 0, st;
         for (int j = i; j < n; j++)
-            if (!done[j] && d[j].A == d[i].A && d[j].K == d[i].K && gemm_f16_takes(d[j].type, M, mode)) {
+            if (!seen[j] && d[j].A == d[i].A && d[j].K == d[i].K) {
+                seen[j] = true;
+                if (!gemm_f16_takes(d[j].type, cols, (int)d[j].K, M, mode)) continue;
                 idx[ng] = j;
                 ge[ng++] = GemmEntry{d[j].W, d[j].type, (int)d[j].N, d[j].C, (int)d[j].N};
             }
-        if (!gemm_f16(c, ar, 0, ge, ng, (int)d[i].K, mode, d[i].A, (int)d[i].K, nullptr, nullptr, M, s, &st)) continue;
+        if (!ng || !gemm_f16(c, ar, 0, ge, ng, (int)d[i].K, mode, d[i].A, (int)d[i].K, nullptr, nullptr, M, s, &st)) continue;
         if (st != GGQ_OK) return st;
         for (int j = 0; j < ng; j++) done[idx[j]] = true;
     }
@@ -342,7 +368,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     g.groups = 1;
     const GemmEntry ge{W, type, (int)N, C, ldc};
     if (act_mode == GGQ_ACT_F32) {
-        if (gemm_f16_takes(type, M, GEMM_F32) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_F32, A, lda, nullptr, nullptr, M, s, &st)) return st;
+        if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_F32, A, lda, nullptr, nullptr, M, s, &st)) return st;
         g.X = A;
         g.ldx = lda;
         return hip_status(c, ggq::launch_gemv(g, s), "gemv");
@@ -360,7 +386,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
         if (ggq::i8_gemv_eligible(&g, 1, 1))
             return hip_status(c, ggq::launch_i8_gemv(&g, 1, 1, nullptr, nullptr, s), "gemv_i8");
     }
-    if (act_mode == GGQ_ACT_Q8_ROW && gemm_f16_takes(type, M, GEMM_Q8_ROW) &&
+    if (act_mode == GGQ_ACT_Q8_ROW && gemm_f16_takes(type, N, (int)K, M, GEMM_Q8_ROW) &&
         gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_Q8_ROW, A, lda, nullptr, nullptr, M, s, &st))
         return st;
     if (act_mode == GGQ_ACT_Q8_ROW && M > 8 && ggq::gemm_panel_eligible(type, (int)K, M, A, lda)) {
@@ -388,7 +414,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     }
     if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, nullptr, nullptr, xe, s)) != hipSuccess)
         return hip_status(c, e, "quant_act");
-    if (gemm_f16_takes(type, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
+    if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
     g.X = xe;
     g.ldx = (int)K;
     return hip_status(c, ggq::launch_gemv(g, s), "gemv");
@@ -403,7 +429,7 @@ int mul_mat_q8_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_
     void* ws;
     float* part;
     const GemmEntry ge{W, type, (int)N, C, ldc};
-    if (gemm_f16_takes(type, M, GEMM_CODES) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_CODES, nullptr, 0, qa, sa, M, s, &st)) return st;
+    if (gemm_f16_takes(type, N, (int)K, M, GEMM_CODES) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_CODES, nullptr, 0, qa, sa, M, s, &st)) return st;
     if (M > 8 && ggq::gemm_panel_eligible(type, (int)K, M, nullptr, 0)) {
         const ggq::GemmDesc gd{W, C, (int)N, ldc};
         return hip_status(c, ggq::launch_gemm_panel(type, &gd, 1, (int)K, nullptr, 0, qa, sa, M, s), "gemm_panel");
@@ -811,7 +837,9 @@ int ggq_mul_mat_q8_batch_dev(ggq_ctx* c, const ggq_gemm_desc* d, int n, uint32_t
     if (M == 0) return set_status(c, GGQ_OK);
     const hipStream_t s = pick_stream(c, stream);
     Arena ar = dev_arena(c, s);
-    if (gemm_f16_takes(type, M, GEMM_CODES)) {
+    int64_t cols = 0;
+    for (int i = 0; i < n; i++) cols += d[i].N;
+    if (gemm_f16_takes(type, cols, (int)K, M, GEMM_CODES)) {
         GemmEntry ge[GGQ_MAX_GEMM_BATCH];
         for (int i = 0; i < n; i++) ge[i] = GemmEntry{d[i].W, type, (int)d[i].N, d[i].C, d[i].ldc};
         int st;
