@@ -742,11 +742,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
 }
 
 // ------------------------------------------------------ activation planes --
-// One workgroup per row (rows from M on: zeros).  A thread takes pieces of 8
-// consecutive values; piece p = 4 g + 2 h + u goes to lane slot 32 h + row %
-// 32 of step 2 g + u.  S: the sums over 32 values, divided by 32, as fp16 hi
-// + lo in one more operand per superblock (hi in lane half 0, lo in 1; sub-
-// block j in element j).
+// A workgroup takes RW rows.  A thread takes pieces of 8 consecutive values of
+// one row; piece p = 4 g + 2 h + u goes to lane slot 32 h + row % 32 of step
+// 2 g + u.  S: the sums over 32 values, divided by 32, as fp16 hi + lo in one
+// more operand per superblock (hi in lane half 0, lo in 1; sub-block j in
+// element j).  Slots of rows from M on stay unwritten: each row is an output
+// row of its own in the products, and those are not stored.
 struct PrepArgs {
     const float* A;
     const int8_t* QA;
@@ -761,96 +762,122 @@ constexpr int kPi[8] = {0, 2, 1, 3, 4, 6, 5, 7};
 
 // MODE 0: fp32 rows as hi + lo; 1: fp32 rows quantized per row to int8 codes
 // (the codes and scales of the row quantizer); 2: given int8 codes.
-template <int MODE, int RP, bool VEC>
-__global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
-    __shared__ float wmax[4];
-    // each XCD takes a contiguous range of rows, so that the 16-byte pieces of
-    // neighbouring rows meet in one L2
-    const int m = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), tid = threadIdx.x, np = a.SB * 32;
+//
+// Neighbouring lanes hold the same piece of RW neighbouring rows, which lie
+// side by side in the planes (16 RW bytes a run; with a row per workgroup each
+// lane's 16 bytes go to another line).  RP pieces a thread stay in registers
+// between the row's maximum and the conversion; longer rows are read twice.
+template <int MODE, int RW, int RP, bool VEC>
+__global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
+    __shared__ float wmax[16 * RW];
+    const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
+    // a row each: an XCD takes a contiguous range of them, so that their pieces
+    // meet in one L2 (the grid is then a multiple of 8)
+    const int wg = RW == 1 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const int m = wg * RW + tid % RW, p0 = tid / RW, ps = blockDim.x / RW, np = a.SB * 32;
+    const int64_t row = (int64_t)(m < a.M ? m : a.M - 1) * (MODE == 2 ? a.K : a.lda);
     const size_t tile = (size_t)(m >> 5) * a.SB;
-    const int r = m & 31;
+    const int r = m & 31, chunk = ps * RP;
     float v[RP][8];
+    auto load = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < RP; i++) {
-        const int k = 8 * (tid + 256 * i);
-        const bool in = m < a.M && k < a.K;
-        // no branch around the loads: places past the row read its start
-        const int64_t at = (int64_t)(m < a.M ? m : 0) * (MODE == 2 ? a.K : a.lda) + (k < a.K ? k : 0);
-        if constexpr (MODE == 2) {
-            const uint2 c = *(const uint2*)(a.QA + at);
+        for (int i = 0; i < RP; i++) {
+            const int k = 8 * (c + p0 + ps * i);
+            const bool in = k < a.K;
+            // no branch around the loads: places past the row read its start
+            const int64_t at = row + (in ? k : 0);
+            if constexpr (MODE == 2) {
+                const uint2 q = *(const uint2*)(a.QA + at);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = (float)(int8_t)((e < 4 ? c.x : c.y) >> (8 * (e & 3)));
-        } else if (VEC) {
-            const float4 x = *(const float4*)(a.A + at), y = *(const float4*)(a.A + at + 4);
-            v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
-            v[i][4] = y.x; v[i][5] = y.y; v[i][6] = y.z; v[i][7] = y.w;
-        } else {
+                for (int e = 0; e < 8; e++) v[i][e] = (float)(int8_t)((e < 4 ? q.x : q.y) >> (8 * (e & 3)));
+            } else if (VEC) {
+                const float4 x = *(const float4*)(a.A + at), y = *(const float4*)(a.A + at + 4);
+                v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
+                v[i][4] = y.x; v[i][5] = y.y; v[i][6] = y.z; v[i][7] = y.w;
+            } else {
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[i][e] = a.A[at + e];
+                for (int e = 0; e < 8; e++) v[i][e] = a.A[at + e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[i][e] = in ? v[i][e] : 0.0f;
+        }
+    };
+    int ex = 0;
+    float inv = 0.0f;
+    if constexpr (MODE == 2) {
+        load(0);
+    } else {
+        float amax = 0.0f;
+        for (int c = 0; c < np; c += chunk) {
+            load(c);
+#pragma unroll
+            for (int i = 0; i < RP; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[i][e]));
         }
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[i][e] = in ? v[i][e] : 0.0f;
-    }
-    int ex = 0;
-    if constexpr (MODE != 2) {
-        float amax = 0.0f;
-#pragma unroll
-        for (int i = 0; i < RP; i++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[i][e]));
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        if ((tid & 63) == 0) wmax[tid >> 6] = amax;
+        for (int off = 32; off >= RW; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        if (lane < RW) wmax[(tid >> 6) * RW + lane] = amax;
         __syncthreads();
-        amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        for (int o = 0; o < waves; o++) amax = fmaxf(amax, wmax[o * RW + tid % RW]);
         if constexpr (MODE == 0) {
             if (amax > 0.0f) {  // the largest magnitude into [2^14, 2^15)
                 int x2;
                 (void)frexpf(amax, &x2);
                 ex = 15 - x2 > 126 ? 126 : 15 - x2;
             }
-            if (tid == 0 && m < a.M) a.rs[m] = ldexpf(1.0f, -ex);
+            if (tid < RW && m < a.M) a.rs[m] = ldexpf(1.0f, -ex);
         } else {
             const float sc = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
-            const float inv = __fdiv_rn(1.0f, sc);
-            if (tid == 0 && m < a.M) a.rs[m] = sc;
-#pragma unroll
-            for (int i = 0; i < RP; i++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[i][e] = (float)to_i8(__fmul_rn(v[i][e], inv));
+            inv = __fdiv_rn(1.0f, sc);
+            if (tid < RW && m < a.M) a.rs[m] = sc;
         }
+        if (np > chunk) load(0);
     }
+    for (int c = 0;;) {
 #pragma unroll
-    for (int i = 0; i < RP; i++) {
-        const int p = tid + 256 * i;
-        if (p >= np) break;
-        h8 hi, lo;
-        float gs = 0.0f;
+        for (int i = 0; i < RP; i++) {
+            const int p = c + p0 + ps * i;
+            if (p >= np || m >= a.M) break;
+            h8 hi, lo;
+            float gs = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const float y = MODE == 0 ? ldexpf(v[i][kPi[e]], ex) : v[i][kPi[e]];
-            hi[e] = (_Float16)y;
-            lo[e] = (_Float16)(y - (float)hi[e]);
-            gs += MODE == 0 ? (float)hi[e] + (float)lo[e] : y;
+            for (int e = 0; e < 8; e++) {
+                const float x = v[i][kPi[e]];
+                const float y = MODE == 0 ? ldexpf(x, ex) : MODE == 1 ? (float)to_i8(__fmul_rn(x, inv)) : x;
+                hi[e] = (_Float16)y;
+                lo[e] = (_Float16)(y - (float)hi[e]);
+                gs += MODE == 0 ? (float)hi[e] + (float)lo[e] : y;
+            }
+            const int g = p >> 2, h = (p >> 1) & 1, u = p & 1;
+            const size_t at = (tile * 16 + 2 * g + u) * 64 + 32 * h + r;
+            a.XH[at] = hi;
+            if constexpr (MODE == 0) a.XL[at] = lo;
+            gs += __shfl_xor(gs, RW, 64);  // the group's four pieces: all of them are in this loop
+            gs += __shfl_xor(gs, 2 * RW, 64);
+            const float y = gs * 0.03125f;
+            const _Float16 sh = (_Float16)y, sl = (_Float16)(y - (float)sh);
+            if (u == 0) a.XS[((tile + (g >> 3)) * 64 + 32 * h + r) * 8 + (g & 7)] = h ? sl : sh;
         }
-        const int g = p >> 2, h = (p >> 1) & 1, u = p & 1;
-        const size_t at = (tile * 16 + 2 * g + u) * 64 + 32 * h + r;
-        a.XH[at] = hi;
-        if constexpr (MODE == 0) a.XL[at] = lo;
-        gs += __shfl_xor(gs, 1, 64);
-        gs += __shfl_xor(gs, 2, 64);
-        const float y = gs * 0.03125f;
-        const _Float16 sh = (_Float16)y, sl = (_Float16)(y - (float)sh);
-        if (u == 0) a.XS[((tile + (g >> 3)) * 64 + 32 * h + r) * 8 + (g & 7)] = h ? sl : sh;
+        c += chunk;
+        if (c >= np) break;
+        load(c);
     }
 }
 
+// Four rows a workgroup from 512 rows on, where that still gives half of the
+// CUs one; below that the time is the launch's and one row's latency, and a
+// row per workgroup spreads it (fp32 rows, one against four: 100 x 2048 5.3,
+// 6.8; 500 x 2048 6.8, 6.7; 1023 x 2048 7.4, 7.2; 1023 x 8192 18.6, 12.0 us).
 template <int MODE, bool VEC>
 void launch_prep_v(const PrepArgs& a, hipStream_t s) {
-    const int rows = (a.M + 127) & ~127, np = a.SB * 32;
-    if (np <= 256) prep_kernel<MODE, 1, VEC><<<rows, 256, 0, s>>>(a);
-    else if (np <= 1024) prep_kernel<MODE, 4, VEC><<<rows, 256, 0, s>>>(a);
-    else prep_kernel<MODE, 16, VEC><<<rows, 256, 0, s>>>(a);
+    const int np = a.SB * 32;  // pieces of a row
+    if (a.M >= 512) {
+        const int wgs = (a.M + 3) / 4;
+        if (np <= 512) prep_kernel<MODE, 4, 2, VEC><<<wgs, np * 2, 0, s>>>(a);
+        else prep_kernel<MODE, 4, 4, VEC><<<wgs, 1024, 0, s>>>(a);
+    } else if (np <= 256) prep_kernel<MODE, 1, 1, VEC><<<(a.M + 7) & ~7, 256, 0, s>>>(a);
+    else prep_kernel<MODE, 1, 4, VEC><<<(a.M + 7) & ~7, 256, 0, s>>>(a);
 }
 template <int MODE>
 void launch_prep(const PrepArgs& a, hipStream_t s) {
@@ -879,8 +906,10 @@ Planes planes_of(int K, int M, bool two) {
 //   gets at most one (64 rows: 16 / 29), then 32 columns (19 / 20);
 //   128-row tiles from the ring otherwise: 128 columns a workgroup from two
 //   workgroups a CU (1023 rows: 52 / 86), 64 columns and two K slices from one
-//   (38 / 98), else four K slices: 32 columns, or 64 x 64 where one weight
-//   plane leaves the LDS reads as the bound (500 rows: 29 and 25).
+//   (38 / 98), else four K slices: 32 columns.  With one weight plane 64 x 64
+//   values a wavefront read half as much from LDS and fit the registers: with
+//   two K slices 128 x 64 (8192 x 2048, 500 rows 56.1 -> 53.5; 2048 x 8192,
+//   1023 rows 128 -> 118, codes 72 -> 68), with four 64 x 64 (29 -> 25).
 // More K slices for longer rows keep the fp32 sums short: error against 64
 // bits at K = 8192 2.4e-7, 2.25e-7, 2.15e-7 with one, two, four (the single-
 // row kernels' 2.35e-7).
@@ -915,8 +944,13 @@ void launch_t(Args& a, int M, hipStream_t s) {
         const dim3 g = tiles(128, 128);
         gemm_f16_ring_kernel<T, AP, 4, 1, 4, 4 / AP><<<g, 256, 0, s>>>(a);
     } else if (m128 * cols32 >= 2 * kCus && a.SB <= 32) {
-        const dim3 g = tiles(64, 128);
-        gemm_f16_ring_kernel<T, AP, 4, 1, 2, 2 / AP><<<g, 256, 0, s>>>(a);
+        if constexpr (Col<T, 2, 2>::kTwo) {
+            const dim3 g = tiles(64, 128);
+            gemm_f16_ring_kernel<T, AP, 4, 1, 2, 2 / AP><<<g, 256, 0, s>>>(a);
+        } else {
+            const dim3 g = tiles(128, 64);
+            gemm_f16_ring_kernel<T, AP, 2, 2, 2, 2 / AP><<<g, 256, 0, s>>>(a);
+        }
     } else if constexpr (Col<T, 2, 2>::kTwo) {
         const dim3 g = tiles(32, 128);
         gemm_f16_ring_kernel<T, AP, 4, 1, 1, 1><<<g, 256, 0, s>>>(a);
