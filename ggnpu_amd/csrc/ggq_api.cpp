@@ -1180,15 +1180,12 @@ static int moe_ffn_f16(ggq_ctx* c, const ggq_moe_params* p, hipStream_t s) {
     else
         e = ggq::launch_moe_gemm(p->down_type, gd, s);
     if (e != hipSuccess) return hip_status(c, e, "moe down");
-    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, shared ? D + nk * H : nullptr, p->shared_w, p->out, s)) !=
+    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, shared ? D + nk * H : nullptr, p->shared_w, p->out,
+                                     ggq::MoePick{sel, p->sel_experts, p->sel_weights}, s)) !=
         hipSuccess)
         return hip_status(c, e, "moe combine");
     c->trace = ggq_moe_trace{GGQ_ACT_F32, T, H, F, E, k, (int)rows, shared ? 1 : 0, grp, tok, pos, G, U, hf, nullptr,
                              nullptr, D, shared ? D + nk * H : nullptr};
-    if (p->sel_experts && (e = hipMemcpyAsync(p->sel_experts, sel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy selection");
-    if (p->sel_weights && (e = hipMemcpyAsync(p->sel_weights, wsel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy weights");
     return set_status(c, GGQ_OK);
 }
 
@@ -1343,15 +1340,12 @@ static int moe_ffn_q8(ggq_ctx* c, const ggq_moe_params* p, hipStream_t s) {
     else if (dn_i8) e = ggq::launch_i8_moe_q8(p->down_type, gd, (int)rows, base + o_it2, s, built);
     else e = ggq::launch_moe_gemm(p->down_type, gd, s);
     if (e != hipSuccess) return hip_status(c, e, "moe down");
-    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, shared ? D + nk * H : nullptr, p->shared_w, p->out, s)) !=
+    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, shared ? D + nk * H : nullptr, p->shared_w, p->out,
+                                     ggq::MoePick{sel, p->sel_experts, p->sel_weights}, s)) !=
         hipSuccess)
         return hip_status(c, e, "moe combine");
     c->trace = ggq_moe_trace{GGQ_ACT_Q8_ROW, T, H, F, E, k, (int)rows, shared ? 1 : 0, grp, tok, pos, G, U, hf, qh,
                              sh, D, shared ? D + nk * H : nullptr};
-    if (p->sel_experts && (e = hipMemcpyAsync(p->sel_experts, sel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy selection");
-    if (p->sel_weights && (e = hipMemcpyAsync(p->sel_weights, wsel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy weights");
     return set_status(c, GGQ_OK);
 }
 
@@ -1514,14 +1508,11 @@ int ggq_moe_ffn_dev(ggq_ctx* c, const ggq_moe_params* p, void* stream) {
         q.N = H; q.K = F; q.X = Hh + nk * F; q.ldx = F; q.ldy = H; q.type = p->down_type; q.W = p->down_shexp; q.Y = Dsh;
         if ((e = ggq::launch_gemv(q, s)) != hipSuccess) return hip_status(c, e, "shared down");
     }
-    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, Dsh, p->shared_w, p->out, s)) != hipSuccess)
+    if ((e = ggq::launch_moe_combine(D, pos, wsel, T, k, H, Dsh, p->shared_w, p->out,
+                                     ggq::MoePick{sel, p->sel_experts, p->sel_weights}, s)) != hipSuccess)
         return hip_status(c, e, "moe combine");
     c->trace = ggq_moe_trace{GGQ_ACT_F32, T, H, F, E, k, (int)(nk + ts), shared ? 1 : 0, grp, tok, pos, G, U, Hh,
                              nullptr, nullptr, D, Dsh};
-    if (p->sel_experts && (e = hipMemcpyAsync(p->sel_experts, sel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy selection");
-    if (p->sel_weights && (e = hipMemcpyAsync(p->sel_weights, wsel, 4 * nk, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_status(c, e, "copy weights");
     return set_status(c, GGQ_OK);
     GGQ_END(c)
 }

@@ -4475,15 +4475,26 @@ hipError_t launch_swiglu(const float* g, const float* u, float* h, int64_t n, hi
     return hipGetLastError();
 }
 
+// The caller's copies of token t's experts and weights, written by the token's
+// first workgroup (top_k <= 64 of its threads): no copies of their own behind
+// the layer (two of them cost 2.8 us after one token, 9.6 after 64).
+__device__ __forceinline__ void pick_out(const MoePick& p, const float* wsel, int t, int topk) {
+    if (blockIdx.x || (int)threadIdx.x >= topk) return;
+    const int at = t * topk + threadIdx.x;
+    if (p.sel_out) p.sel_out[at] = p.sel[at];
+    if (p.w_out) p.w_out[at] = wsel[at];
+}
+
 // Weighted combine in the reference's order (main.cpp:3166-3193): routed
 // experts j = 0..topk-1 by descending logit, then the shared expert.
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ D, const int32_t* __restrict__ pos_of,
                                                           const float* __restrict__ wsel, int topk, int H,
                                                           const float* __restrict__ Dsh,
                                                           const float* __restrict__ shared_w,
-                                                          float* __restrict__ out) {
+                                                          float* __restrict__ out, MoePick pick) {
     const int t = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    pick_out(pick, wsel, t, topk);
     if (i >= H) return;
     float acc = 0.0f;
     for (int j = 0; j < topk; j++)
@@ -4493,40 +4504,53 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
 }
 
 // The same with 4 values a thread (16-byte loads and stores; H % 4 == 0,
-// 16-byte aligned rows).
+// 16-byte aligned rows).  A token's rows are loaded eight at a time, in flight
+// together (one after another they cost a memory latency each).
 __global__ __launch_bounds__(256) void moe_combine4_kernel(const float* __restrict__ D, const int32_t* __restrict__ pos_of,
                                                            const float* __restrict__ wsel, int topk, int H,
                                                            const float* __restrict__ Dsh,
                                                            const float* __restrict__ shared_w,
-                                                           float* __restrict__ out) {
+                                                           float* __restrict__ out, MoePick pick) {
     const int t = blockIdx.y;
     const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+    pick_out(pick, wsel, t, topk);
     if (i >= H) return;
+    float4 sh = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (Dsh) sh = *(const float4*)(Dsh + (int64_t)t * H + i);
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int j = 0; j < topk; j++) {
-        const float w = wsel[t * topk + j];
-        const float4 v = *(const float4*)(D + (int64_t)pos_of[t * topk + j] * H + i);
-        acc.x += w * v.x; acc.y += w * v.y; acc.z += w * v.z; acc.w += w * v.w;
+    for (int j0 = 0; j0 < topk; j0 += 8) {
+        float4 v[8];
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int at = t * topk + (j0 + j < topk ? j0 + j : topk - 1);
+            w[j] = wsel[at];
+            v[j] = *(const float4*)(D + (int64_t)pos_of[at] * H + i);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (j0 + j >= topk) break;
+            acc.x += w[j] * v[j].x; acc.y += w[j] * v[j].y; acc.z += w[j] * v[j].z; acc.w += w[j] * v[j].w;
+        }
     }
     if (Dsh) {
         const float w = shared_w ? shared_w[t] : 1.0f;
-        const float4 v = *(const float4*)(Dsh + (int64_t)t * H + i);
-        acc.x += w * v.x; acc.y += w * v.y; acc.z += w * v.z; acc.w += w * v.w;
+        acc.x += w * sh.x; acc.y += w * sh.y; acc.z += w * sh.z; acc.w += w * sh.w;
     }
     *(float4*)(out + (int64_t)t * H + i) = acc;
 }
 
 hipError_t launch_moe_combine(const float* D, const int32_t* pos_of, const float* wsel, int T,
                               int topk, int H, const float* Dsh, const float* shared_w, float* out,
-                              hipStream_t s) {
+                              const MoePick& pick, hipStream_t s) {
     if (T == 0) return hipSuccess;
     const bool v4 = H % 4 == 0 && ((uintptr_t)D & 15u) == 0 && ((uintptr_t)out & 15u) == 0 &&
                     (!Dsh || ((uintptr_t)Dsh & 15u) == 0);
     if (v4) {
-        moe_combine4_kernel<<<dim3((H / 4 + 255) / 256, T), 256, 0, s>>>(D, pos_of, wsel, topk, H, Dsh, shared_w, out);
+        moe_combine4_kernel<<<dim3((H / 4 + 255) / 256, T), 256, 0, s>>>(D, pos_of, wsel, topk, H, Dsh, shared_w, out, pick);
         return hipGetLastError();
     }
-    moe_combine_kernel<<<dim3((H + 255) / 256, T), 256, 0, s>>>(D, pos_of, wsel, topk, H, Dsh, shared_w, out);
+    moe_combine_kernel<<<dim3((H + 255) / 256, T), 256, 0, s>>>(D, pos_of, wsel, topk, H, Dsh, shared_w, out, pick);
     return hipGetLastError();
 }
 

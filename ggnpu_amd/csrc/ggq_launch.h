@@ -267,8 +267,15 @@ ChunkList i8_moe_q8_list(uint32_t type, const MoeGemm& g, int rows, void* ws);
 hipError_t launch_split_rows(int producer, const float* A, const float* aux, int lda, int M, int K, void* XH,
                              void* XL, float* XS, float* xs, float* prod_out, hipStream_t s);
 hipError_t launch_swiglu(const float* g, const float* u, float* h, int64_t n, hipStream_t s);
+// Weighted sum of a token's expert rows; also writes the caller's copies of
+// the selection and its weights, where asked for.
+struct MoePick {
+    const int32_t* sel;
+    int32_t* sel_out;  // [T][topk] or null
+    float* w_out;      // [T][topk] or null
+};
 hipError_t launch_moe_combine(const float* D, const int32_t* pos_of, const float* wsel, int T,
                               int topk, int H, const float* Dsh, const float* shared_w, float* out,
-                              hipStream_t s);
+                              const MoePick& pick, hipStream_t s);
 
 }  // namespace ggq
