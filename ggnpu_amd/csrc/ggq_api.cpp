@@ -280,13 +280,59 @@ bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
     const bool blocks32 = type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL;
     const int64_t w = cols * K, work = w * M;
     if (mode == GEMM_F32) {
-        if (blocks32) return M >= 48 && work >= (int64_t)256 << 20;
-        return work >= (w >= 1 << 22 ? (int64_t)80 << 20 : (int64_t)256 << 20);
+        // (the wavefronts of few columns take long K in turn: 333 x 16384 Q4_K,
+        // 48 rows 36 -> 71, Q8_0, 64 rows 49 -> 84)
+        if (blocks32) return M >= 48 && cols * M >= 49152 && work >= (int64_t)256 << 20;
+        return cols * M >= 32768 && work >= (w >= 1 << 22 ? (int64_t)80 << 20 : (int64_t)256 << 20);
     }
     if (type == GGQ_TYPE_Q6_K) return true;
     if (blocks32) return false;
     if (K <= 2048) return true;
     return type != GGQ_TYPE_IQ4_XS && (M <= 32 || M > 64);
+}
+
+// What the register-resident kernel of few fp32 rows takes: `types` formats in
+// the group of matmuls, which it multiplies in one launch where the GEMM above
+// needs one each.  It wins where the weights outweigh its start (each CU loads
+// and splits all rows of its superblocks once): us before -> there, Q4_K / Q6_K:
+//   8 rows: 2048 x 2048 7.8 -> 7.9 / 8.1 -> 7.9, 8192 x 2048 14.6 -> 9.5 / 15.1
+//   -> 9.8, 32000 x 2048 39 -> 17 / 42 -> 20 (up to 4 rows the GEMVs keep up);
+//   16 rows: 512 x 2048 5.9 -> 7.7 / 6.0 -> 7.7, 1024 x 3072 11.3 -> 9.2 / 11.2
+//   -> 9.4, 16384 x 2048 20 -> 12 / 24 -> 13;
+//   32 rows: 6144 x 1024 9.5 -> 11.5 / 11.9 -> 10.7, 2048 x 2048 11.4 -> 11.5 /
+//   12.5 -> 10.5, 16384 x 2048 25 -> 17 / 30 -> 18, 2048 x 8192 23 -> 17 / 28 ->
+//   17 (its 32-row splitting also sums the K-quants' groups).
+//   Q8_0 and IQ4_NL blocks load as in the GEMM: 8192 x 2048, 12 / 16 / 32 rows
+//   18 -> 18, 20 -> 18, 30 -> 21.
+constexpr int kRowsMin = 5;
+bool gemm_rows_takes(uint32_t type, int64_t cols, int K, int M, int types) {
+    if (M < kRowsMin || M > 32) return false;
+    const int64_t w = cols * K, mi = 1 << 20;
+    if (type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL) return w >= 16 * mi && (M >= 16 || (K > 2048 && M > 8));
+    if (M <= 8) return w >= 8 * mi && w * M >= 48 * mi;
+    if (M < 12 && cols < 512) return false;
+    if (M > 16 && types == 1 && K <= 4096 && (type == GGQ_TYPE_Q4_K || type == GGQ_TYPE_Q5_K)) return w >= 8 * mi;
+    return w >= 3 * mi;
+}
+
+// Queued on that kernel: true (*st the status); false: left to the others.
+bool gemm_rows(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n, int K, const float* A, int lda, int M,
+               hipStream_t s, int* st) {
+    if (!ggq::gemm_rows_eligible(K, M, A, lda)) return false;
+    int64_t cols = 0;
+    for (int i = 0; i < n; i++) cols += d[i].N;
+    if (cols > INT32_MAX) return false;
+    const size_t bytes = ggq::gemm_rows_ws_bytes(K, M, cols);
+    void* ws = bytes ? ar.planes(ws_bytes, bytes) : nullptr;
+    if (bytes && !ws) return false;
+    ggq::GemmDesc gd[GGQ_MAX_BATCH];
+    uint32_t types[GGQ_MAX_BATCH];
+    for (int i = 0; i < n; i++) {
+        gd[i] = ggq::GemmDesc{d[i].W, d[i].C, d[i].N, d[i].ldc};
+        types[i] = d[i].type;
+    }
+    *st = hip_status(c, ggq::launch_gemm_rows(gd, types, n, K, A, lda, M, ws, s), "gemm_rows");
+    return true;
 }
 
 // Rows per pass over the weights: the planes of a pass stay within 256 MB.
@@ -333,10 +379,28 @@ int gemm_f16_shared(ggq_ctx* c, Arena& ar, const ggq_gemv_desc* d, int n, int M,
     for (int i = 0; i < n; i++) {
         if (seen[i]) continue;
         int64_t cols = 0;
+        int types = 0;
         for (int j = i; j < n; j++)
-            if (d[j].A == d[i].A && d[j].K == d[i].K) cols += d[j].N;
+            if (d[j].A == d[i].A && d[j].K == d[i].K) {
+                cols += d[j].N;
+                bool first = true;
+                for (int k = i; k < j; k++) first = first && !(d[k].A == d[i].A && d[k].K == d[i].K && d[k].type == d[j].type);
+                types += first;
+            }
         GemmEntry ge[GGQ_MAX_BATCH];
         int idx[GGQ_MAX_BATCH], ng = 0, st;
+        if (mode == GEMM_F32) {
+            for (int j = i; j < n; j++)
+                if (d[j].A == d[i].A && d[j].K == d[i].K && gemm_rows_takes(d[j].type, cols, (int)d[j].K, M, types)) {
+                    idx[ng] = j;
+                    ge[ng++] = GemmEntry{d[j].W, d[j].type, (int)d[j].N, d[j].C, (int)d[j].N};
+                }
+            if (ng && gemm_rows(c, ar, 0, ge, ng, (int)d[i].K, d[i].A, (int)d[i].K, M, s, &st)) {
+                if (st != GGQ_OK) return st;
+                for (int j = 0; j < ng; j++) done[idx[j]] = seen[idx[j]] = true;
+            }
+            ng = 0;
+        }
         for (int j = i; j < n; j++)
             if (!seen[j] && d[j].A == d[i].A && d[j].K == d[i].K) {
                 seen[j] = true;
@@ -368,6 +432,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     g.groups = 1;
     const GemmEntry ge{W, type, (int)N, C, ldc};
     if (act_mode == GGQ_ACT_F32) {
+        if (gemm_rows_takes(type, N, (int)K, M, 1) && gemm_rows(c, ar, 0, &ge, 1, (int)K, A, lda, M, s, &st)) return st;
         if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_F32, A, lda, nullptr, nullptr, M, s, &st)) return st;
         g.X = A;
         g.ldx = lda;
@@ -414,6 +479,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     }
     if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, nullptr, nullptr, xe, s)) != hipSuccess)
         return hip_status(c, e, "quant_act");
+    if (gemm_rows_takes(type, N, (int)K, M, 1) && gemm_rows(c, ar, need, &ge, 1, (int)K, xe, (int)K, M, s, &st)) return st;
     if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
     g.X = xe;
     g.ldx = (int)K;
@@ -893,7 +959,7 @@ int ggq_mul_mat_batch_rows_dev(ggq_ctx* c, const ggq_gemv_desc* d, int n, int M,
     if (M == 0) return set_status(c, GGQ_OK);
     const hipStream_t s = pick_stream(c, stream);
     bool done[GGQ_MAX_BATCH] = {};
-    if (M >= kGemmMinRows) {
+    if (M >= kRowsMin) {
         Arena ar = dev_arena(c, s);
         const int st = gemm_f16_shared(c, ar, d, n, M, GEMM_F32, s, done);
         if (st != GGQ_OK) return st;

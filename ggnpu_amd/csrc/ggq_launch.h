@@ -158,6 +158,14 @@ hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t*
                                 hipStream_t s);
 hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, bool codes, const float* sa,
                            const void* ws, hipStream_t s);
+// The same products for few fp32 rows (1..32, A 16-byte aligned, lda % 4 ==
+// 0), which are split in registers, not in planes (ggq_gemm_rows.hip): up to 8
+// weights of any types in one launch.  `ws`: gemm_rows_ws_bytes(K, M, columns
+// of all weights) bytes, none up to K = 2048.
+bool gemm_rows_eligible(int K, int M, const float* A, int lda);
+size_t gemm_rows_ws_bytes(int K, int M, int64_t cols);
+hipError_t launch_gemm_rows(const GemmDesc* d, const uint32_t* types, int n, int K, const float* A, int lda, int M, void* ws,
+                            hipStream_t s);
 // idx[m] = first index of the largest value of row m of L ([M][ld], N
 // values); val[m] = that value (val may be null).  `ws`: device workspace
 // of argmax_workspace_bytes(M) bytes.
