@@ -1164,6 +1164,16 @@ static bool moe_small_groups(size_t rows, int groups, int dflt = 5) {
     return rows <= max_avg * (size_t)groups;
 }
 
+// Whether one launch does everything behind gate and up: it reads the weights
+// of every pair row, so it wins while the launches it saves outweigh what
+// tokens could share (Q4_K, Q4_K, Q6_K, us before -> there): one token 38.6 ->
+// 28.5 (256 experts, top 8, F = 512), 27.9 -> 26.3 (64, 2, 2048); two 46.8 ->
+// 40.9, but 44.4 -> 45.4 with F = 768; four 33.9 -> 32.0 (32, 4, 256), but 48 ->
+// 60 (256, 8, 512).
+static bool moe_down_takes(uint32_t type, int T, int k, int F) {
+    return (T == 1 || (T <= 4 && T * k * F <= 8192)) && ggq::moe_down_eligible(type, F, k);
+}
+
 // MoE layer with fp32 activations at prefill-sized batches: route, group
 // (tile list over the experts and the shared expert as group E), the token
 // rows split once into fp16 hi + lo planes, one expert-grouped fp16 GEMM
@@ -1549,6 +1559,21 @@ int ggq_moe_ffn_dev(ggq_ctx* c, const ggq_moe_params* p, void* stream) {
             q.type = p->up_type; q.W = p->up_shexp; q.Y = SU;
             if ((e = ggq::launch_gemv(q, s)) != hipSuccess) return hip_status(c, e, "shared up");
         }
+    }
+    // Few tokens: everything behind gate and up in one launch.
+    if (moe_down_takes(p->down_type, T, k, F)) {
+        ggq::MoeDown m{};
+        m.W = (const uint8_t*)p->down_exps;
+        m.w_stride = (int64_t)H * ggq::row_bytes(p->down_type, F);
+        m.Wsh = (const uint8_t*)p->down_shexp;
+        m.G = G; m.U = U; m.Hh = Hh; m.D = D; m.Dsh = Dsh;
+        m.pos = pos; m.wsel = wsel; m.shared_w = p->shared_w; m.out = p->out;
+        m.pick = ggq::MoePick{sel, p->sel_experts, p->sel_weights};
+        m.T = T; m.H = H; m.F = F; m.E = E; m.topk = k;
+        if ((e = ggq::launch_moe_down(p->down_type, m, s)) != hipSuccess) return hip_status(c, e, "moe down");
+        c->trace = ggq_moe_trace{GGQ_ACT_F32, T, H, F, E, k, (int)(nk + ts), shared ? 1 : 0, grp, tok, pos, G, U, Hh,
+                                 nullptr, nullptr, D, Dsh};
+        return set_status(c, GGQ_OK);
     }
     // SwiGLU of the routed pair rows and the shared expert's rows together.
     if ((e = ggq::launch_swiglu(G, U, Hh, (int64_t)(nk + ts) * F, s)) != hipSuccess) return hip_status(c, e, "swiglu");

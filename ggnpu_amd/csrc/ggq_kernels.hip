@@ -4554,4 +4554,130 @@ hipError_t launch_moe_combine(const float* D, const int32_t* pos_of, const float
     return hipGetLastError();
 }
 
+// The rest of a layer behind gate and up for few tokens: SwiGLU, the routed
+// and the shared expert's down projection and the weighted sum, in one launch.
+// A workgroup takes kDownCols columns of a token, a wavefront an expert of its
+// selection (then the shared expert): it makes the SwiGLU row from G and U in
+// registers, a piece of 32 values a lane, and its column sums meet in LDS,
+// where they are added in the order of moe_combine_kernel.  A token's layer is
+// latency: four launches (SwiGLU 2.3, the grouped GEMV over a grid of every
+// expert 11.4, the shared expert's 3.8, combine 3 us and the gaps) become one
+// (256 experts, top 8, F = 512, Q4_K / Q6_K: the layer 38.6 -> 28.5 us).
+constexpr int kDownCols = 8;
+template <int T, int U>
+__global__ __launch_bounds__(1024) void moe_down_kernel(MoeDown a) {
+    __shared__ float part[65][kDownCols];
+    const int t = blockIdx.y, n0 = blockIdx.x * kDownCols;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int lg = a.lpr_log2, lp = lane & ((1 << lg) - 1), rsub = lane >> lg, rpi = 64 >> lg;
+    const int P = a.F >> 5, pairs = a.topk + (a.Dsh ? 1 : 0);
+    const bool ok = lp < P;
+    const int p = ok ? lp : 0;
+    pick_out(a.pick, a.wsel, t, a.topk);
+    for (int j = wave; j < pairs; j += waves) {
+        const uint8_t* W = a.Wsh;
+        int64_t hrow = (int64_t)a.T * a.topk + t;
+        float* d = a.Dsh + (int64_t)t * a.H;
+        if (j < a.topk) {
+            W = a.W + expert_id(a.pick.sel[t * a.topk + j], a.E) * a.w_stride;
+            hrow = a.pos[t * a.topk + j];
+            d = a.D + hrow * a.H;
+        }
+        auto row = [&](int it) {
+            const int n = n0 + it * rpi + rsub;
+            return make_row(W, (uint32_t)(n < a.H ? n : a.H - 1) * a.row_bytes);
+        };
+        typename Piece<T>::Raw raw[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) raw[u] = Piece<T>::fetch(row(u), p);
+        float x[32], xs[2];
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int64_t at = hrow * a.F + Piece<T>::run_k(p, r);
+            float4 g[4], u[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                g[c] = *(const float4*)(a.G + at + 4 * c);
+                u[c] = *(const float4*)(a.U + at + 4 * c);
+            }
+            xs[r] = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                float4 h;
+                h.x = (g[c].x / (1.0f + expf(-g[c].x))) * u[c].x;
+                h.y = (g[c].y / (1.0f + expf(-g[c].y))) * u[c].y;
+                h.z = (g[c].z / (1.0f + expf(-g[c].z))) * u[c].z;
+                h.w = (g[c].w / (1.0f + expf(-g[c].w))) * u[c].w;
+                if (n0 == 0 && rsub == 0 && ok) *(float4*)(a.Hh + at + 4 * c) = h;
+                x[16 * r + 4 * c] = ok ? h.x : 0.0f;
+                x[16 * r + 4 * c + 1] = ok ? h.y : 0.0f;
+                x[16 * r + 4 * c + 2] = ok ? h.z : 0.0f;
+                x[16 * r + 4 * c + 3] = ok ? h.w : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) xs[r] += x[16 * r + i];
+        }
+        for (int it = 0; it * rpi < kDownCols; it += U) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const PieceCodes pc = Piece<T>::decode(raw[u], row(it + u), p);
+                float v = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    float f[16], s0 = 0.0f, s1 = 0.0f;
+                    ubytes_to_f32(pc.u[r], f);
+#pragma unroll
+                    for (int i = 0; i < 16; i += 2) {
+                        s0 = fmaf(x[16 * r + i], f[i], s0);
+                        s1 = fmaf(x[16 * r + i + 1], f[i + 1], s1);
+                    }
+                    v = fmaf(pc.a[r], s0 + s1, fmaf(pc.b[r], xs[r], v));
+                }
+                v = group_sum(v, lg);
+                const int c = (it + u) * rpi + rsub;
+                if (lp == 0) {
+                    part[j][c] = v;
+                    if (n0 + c < a.H) d[n0 + c] = v;
+                }
+                if ((it + U) * rpi < kDownCols) raw[u] = Piece<T>::fetch(row(it + U + u), p);
+            }
+        }
+    }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c >= kDownCols || n0 + c >= a.H) return;
+    float acc = 0.0f;
+    for (int j = 0; j < a.topk; j++) acc += a.wsel[t * a.topk + j] * part[j][c];
+    if (a.Dsh) acc += (a.shared_w ? a.shared_w[t] : 1.0f) * part[a.topk][c];
+    a.out[(int64_t)t * a.H + n0 + c] = acc;
+}
+
+bool moe_down_eligible(uint32_t type, int F, int topk) { return supported(type) && F % 32 == 0 && F <= 2048 && topk <= 64; }
+
+hipError_t launch_moe_down(uint32_t type, MoeDown a, hipStream_t s) {
+    if (!moe_down_eligible(type, a.F, a.topk) || a.T < 1) return hipErrorInvalidValue;
+    a.row_bytes = (uint32_t)row_bytes(type, a.F);
+    a.lpr_log2 = 3;
+    while (1 << a.lpr_log2 < a.F / 32) a.lpr_log2++;
+    const int pairs = a.topk + (a.Dsh ? 1 : 0), its = kDownCols >> (6 - a.lpr_log2);
+    const dim3 grid((a.H + kDownCols - 1) / kDownCols, a.T), block(64 * (pairs < 16 ? pairs : 16));
+#define GO(TT)                                                            \
+    case TT:                                                              \
+        if (its == 1) moe_down_kernel<TT, 1><<<grid, block, 0, s>>>(a);   \
+        else if (its == 2) moe_down_kernel<TT, 2><<<grid, block, 0, s>>>(a); \
+        else moe_down_kernel<TT, 4><<<grid, block, 0, s>>>(a);            \
+        break
+    switch (type) {
+        GO(T_Q4_K);
+        GO(T_Q5_K);
+        GO(T_Q6_K);
+        GO(T_Q8_0);
+        GO(T_IQ4_NL);
+        GO(T_IQ4_XS);
+    default: return hipErrorInvalidValue;
+    }
+#undef GO
+    return hipGetLastError();
+}
+
 }  // namespace ggq

@@ -285,5 +285,25 @@ struct MoePick {
 hipError_t launch_moe_combine(const float* D, const int32_t* pos_of, const float* wsel, int T,
                               int topk, int H, const float* Dsh, const float* shared_w, float* out,
                               const MoePick& pick, hipStream_t s);
+// SwiGLU, down projections (routed and shared) and weighted sum of few tokens
+// in one launch: G, U [T topk + T][F] (pair rows pos, then the shared rows),
+// all written as by the separate launches (Hh, D, Dsh, out, pick); F a multiple
+// of 32 up to 2048, rows 16-byte aligned.
+struct MoeDown {
+    const uint8_t* W;
+    int64_t w_stride;
+    const uint8_t* Wsh;
+    const float *G, *U;
+    float *Hh, *D, *Dsh;
+    const int32_t* pos;
+    const float *wsel, *shared_w;
+    float* out;
+    MoePick pick;
+    int T, H, F, E, topk;
+    uint32_t row_bytes;  // these two set by the launch
+    int lpr_log2;
+};
+bool moe_down_eligible(uint32_t type, int F, int topk);
+hipError_t launch_moe_down(uint32_t type, MoeDown a, hipStream_t s);
 
 }  // namespace ggq
