@@ -291,10 +291,20 @@ bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
     return type != GGQ_TYPE_IQ4_XS && (M <= 32 || M > 64);
 }
 
-// What the register-resident kernel of few fp32 rows takes: `types` formats in
-// the group of matmuls, which it multiplies in one launch where the GEMM above
-// needs one each.  It wins where the weights outweigh its start (each CU loads
-// and splits all rows of its superblocks once): us before -> there, Q4_K / Q6_K:
+// What a group of matmuls that share their rows is, for the rule below.
+struct GroupShape {
+    int64_t cols = 0;
+    uint32_t types = 0;  // a bit per format
+    int n_types() const { return __builtin_popcount(types); }
+    static bool blocks32(uint32_t type) { return type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL; }
+    void add(uint32_t type, int64_t n) { cols += n; types |= 1u << type; }
+};
+
+// Whether the register-resident kernel of few fp32 rows takes a group, all of
+// its formats in one launch (the kernels below need one each, the GEMVs of
+// mixed formats one per kind).  It wins where the weights outweigh its start:
+// each CU loads and splits all rows of its superblocks once.  us before ->
+// there, Q4_K / Q6_K:
 //   8 rows: 2048 x 2048 7.8 -> 7.9 / 8.1 -> 7.9, 8192 x 2048 14.6 -> 9.5 / 15.1
 //   -> 9.8, 32000 x 2048 39 -> 17 / 42 -> 20 (up to 4 rows the GEMVs keep up);
 //   16 rows: 512 x 2048 5.9 -> 7.7 / 6.0 -> 7.7, 1024 x 3072 11.3 -> 9.2 / 11.2
@@ -304,15 +314,30 @@ bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
 //   17 (its 32-row splitting also sums the K-quants' groups).
 //   Q8_0 and IQ4_NL blocks load as in the GEMM: 8192 x 2048, 12 / 16 / 32 rows
 //   18 -> 18, 20 -> 18, 30 -> 21.
+//   q/k/v of mixed formats: Q4_K + Q6_K, 3072 x 1024, 5 / 9 / 32 rows 6.2 -> 6.1,
+//   8.2 -> 6.1, 12 -> 9, 4096 x 1024, 5 rows 7.1 -> 6.2; with IQ4_NL, 3072 x 1024
+//   6.0 -> 7.6, 8.1 -> 7.6, 12 -> 9.5, 3072 x 2048 9.7 -> 13.7, 12 -> 14, 20 ->
+//   16, 8208 x 1536 16 -> 13, 18 -> 13, 36 -> 17.
 constexpr int kRowsMin = 5;
-bool gemm_rows_takes(uint32_t type, int64_t cols, int K, int M, int types) {
+bool gemm_rows_takes(const GroupShape& g, int K, int M) {
     if (M < kRowsMin || M > 32) return false;
-    const int64_t w = cols * K, mi = 1 << 20;
-    if (type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL) return w >= 16 * mi && (M >= 16 || (K > 2048 && M > 8));
-    if (M <= 8) return w >= 8 * mi && w * M >= 48 * mi;
-    if (M < 12 && cols < 512) return false;
-    if (M > 16 && types == 1 && K <= 4096 && (type == GGQ_TYPE_Q4_K || type == GGQ_TYPE_Q5_K)) return w >= 8 * mi;
-    return w >= 3 * mi;
+    const int64_t w = g.cols * K, mi = 1 << 20;
+    const bool mixed = g.n_types() > 1;
+    if (g.types & (1u << GGQ_TYPE_Q8_0 | 1u << GGQ_TYPE_IQ4_NL)) {
+        if (!mixed) return w >= 16 * mi && (M >= 16 || (K > 2048 && M > 8));
+        if (M <= 8) return w >= 12 * mi && w < 24 * mi;
+        return w >= 12 * mi || (w >= 3 * mi && ((K < 2048 && M <= 16) || M >= 24));
+    }
+    if (M <= 8) return mixed ? w >= 4 * mi : w >= 8 * mi && w * M >= 48 * mi;
+    if (M < 12 && g.cols < 512) return false;
+    const bool one_plane = !(g.types & ~(1u << GGQ_TYPE_Q4_K | 1u << GGQ_TYPE_Q5_K));
+    if (M > 16 && !mixed && K <= 4096 && one_plane) return w >= 8 * mi;
+    return w >= (mixed && M <= 16 ? 2 : 3) * mi;
+}
+bool gemm_rows_takes(uint32_t type, int64_t N, int K, int M) {
+    GroupShape g;
+    g.add(type, N);
+    return gemm_rows_takes(g, K, M);
 }
 
 // Queued on that kernel: true (*st the status); false: left to the others.
@@ -378,37 +403,49 @@ int gemm_f16_shared(ggq_ctx* c, Arena& ar, const ggq_gemv_desc* d, int n, int M,
     bool seen[GGQ_MAX_BATCH] = {};
     for (int i = 0; i < n; i++) {
         if (seen[i]) continue;
-        int64_t cols = 0;
-        int types = 0;
+        // all: every entry that shares the rows; big: those of 256-value blocks
+        GroupShape all, big;
         for (int j = i; j < n; j++)
-            if (d[j].A == d[i].A && d[j].K == d[i].K) {
-                cols += d[j].N;
-                bool first = true;
-                for (int k = i; k < j; k++) first = first && !(d[k].A == d[i].A && d[k].K == d[i].K && d[k].type == d[j].type);
-                types += first;
+            if (!seen[j] && d[j].A == d[i].A && d[j].K == d[i].K) {
+                all.add(d[j].type, d[j].N);
+                if (!GroupShape::blocks32(d[j].type)) big.add(d[j].type, d[j].N);
             }
+        const int K = (int)d[i].K;
+        const bool large = all.cols * K >= (int64_t)24 << 20;  // a launch more or less does not matter
         GemmEntry ge[GGQ_MAX_BATCH];
         int idx[GGQ_MAX_BATCH], ng = 0, st;
         if (mode == GEMM_F32) {
+            const bool whole = gemm_rows_takes(all, K, M);
             for (int j = i; j < n; j++)
-                if (d[j].A == d[i].A && d[j].K == d[i].K && gemm_rows_takes(d[j].type, cols, (int)d[j].K, M, types)) {
+                if (!seen[j] && d[j].A == d[i].A && d[j].K == d[i].K &&
+                    (whole || (large && !GroupShape::blocks32(d[j].type) && gemm_rows_takes(big, K, M)))) {
                     idx[ng] = j;
                     ge[ng++] = GemmEntry{d[j].W, d[j].type, (int)d[j].N, d[j].C, (int)d[j].N};
                 }
-            if (ng && gemm_rows(c, ar, 0, ge, ng, (int)d[i].K, d[i].A, (int)d[i].K, M, s, &st)) {
+            if (ng && gemm_rows(c, ar, 0, ge, ng, K, d[i].A, K, M, s, &st)) {
                 if (st != GGQ_OK) return st;
                 for (int j = 0; j < ng; j++) done[idx[j]] = seen[idx[j]] = true;
             }
             ng = 0;
         }
+        int refused = 0;
         for (int j = i; j < n; j++)
             if (!seen[j] && d[j].A == d[i].A && d[j].K == d[i].K) {
                 seen[j] = true;
-                if (!gemm_f16_takes(d[j].type, cols, (int)d[j].K, M, mode)) continue;
+                if (!gemm_f16_takes(d[j].type, all.cols, K, M, mode)) {
+                    refused++;
+                    continue;
+                }
                 idx[ng] = j;
                 ge[ng++] = GemmEntry{d[j].W, d[j].type, (int)d[j].N, d[j].C, (int)d[j].N};
             }
-        if (!ng || !gemm_f16(c, ar, 0, ge, ng, (int)d[i].K, mode, d[i].A, (int)d[i].K, nullptr, nullptr, M, s, &st)) continue;
+        // fp32 rows: a launch per format against the GEMVs', which multiply mixed
+        // formats together, so a group stays with them as a whole where it has a
+        // member that does, and a small one always (Q4_K + Q6_K, 3072 x 2048, 40
+        // rows 21 -> 28 us)
+        const bool small = all.n_types() > 1 && all.cols * K < (int64_t)8 << 20;
+        if (mode == GEMM_F32 && ((refused && !large) || small)) ng = 0;
+        if (!ng || !gemm_f16(c, ar, 0, ge, ng, K, mode, d[i].A, K, nullptr, nullptr, M, s, &st)) continue;
         if (st != GGQ_OK) return st;
         for (int j = 0; j < ng; j++) done[idx[j]] = true;
     }
@@ -432,7 +469,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     g.groups = 1;
     const GemmEntry ge{W, type, (int)N, C, ldc};
     if (act_mode == GGQ_ACT_F32) {
-        if (gemm_rows_takes(type, N, (int)K, M, 1) && gemm_rows(c, ar, 0, &ge, 1, (int)K, A, lda, M, s, &st)) return st;
+        if (gemm_rows_takes(type, N, (int)K, M) && gemm_rows(c, ar, 0, &ge, 1, (int)K, A, lda, M, s, &st)) return st;
         if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, 0, &ge, 1, (int)K, GEMM_F32, A, lda, nullptr, nullptr, M, s, &st)) return st;
         g.X = A;
         g.ldx = lda;
@@ -479,7 +516,7 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
     }
     if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, nullptr, nullptr, xe, s)) != hipSuccess)
         return hip_status(c, e, "quant_act");
-    if (gemm_rows_takes(type, N, (int)K, M, 1) && gemm_rows(c, ar, need, &ge, 1, (int)K, xe, (int)K, M, s, &st)) return st;
+    if (gemm_rows_takes(type, N, (int)K, M) && gemm_rows(c, ar, need, &ge, 1, (int)K, xe, (int)K, M, s, &st)) return st;
     if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
     g.X = xe;
     g.ldx = (int)K;
