@@ -1203,12 +1203,12 @@ static bool moe_small_groups(size_t rows, int groups, int dflt = 5) {
 
 // Whether one launch does everything behind gate and up: it reads the weights
 // of every pair row, so it wins while the launches it saves outweigh what
-// tokens could share (Q4_K, Q4_K, Q6_K, us before -> there): one token 38.6 ->
-// 28.5 (256 experts, top 8, F = 512), 27.9 -> 26.3 (64, 2, 2048); two 46.8 ->
-// 40.9, but 44.4 -> 45.4 with F = 768; four 33.9 -> 32.0 (32, 4, 256), but 48 ->
-// 60 (256, 8, 512).
+// tokens could share (Q4_K, Q4_K, Q6_K, us before -> there): one token 38.4 ->
+// 25.2 (256 experts, top 8, F = 512), 27.9 -> 25.9 (64, 2, 2048); two 43.9 ->
+// 43.2 (128, 8, 768), three there 47.8 -> 54.7; four 48.0 -> 47.0 (256, 8, 512),
+// six 64 -> 70; eight 34.6 -> 29.5 (32, 4, 256).
 static bool moe_down_takes(uint32_t type, int T, int k, int F) {
-    return (T == 1 || (T <= 4 && T * k * F <= 8192)) && ggq::moe_down_eligible(type, F, k);
+    return (T == 1 || (T <= 8 && T * k * F <= 16384)) && ggq::moe_down_eligible(type, F, k);
 }
 
 // MoE layer with fp32 activations at prefill-sized batches: route, group

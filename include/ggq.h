@@ -85,7 +85,9 @@ int ggq_sync(ggq_ctx* ctx);
  * made while its stream is being captured never allocates: if its workspace
  * is too small it fails with GGQ_ERROR and says so in
  * ggq_last_error_message.  Size the workspace before a capture by running
- * the captured calls once outside it, or with ggq_reserve.  The synchronous
+ * the captured calls once outside it, or with ggq_reserve.  Matmuls of 5 rows
+ * and more also use a buffer per stream (at most 8 streams), and kernels that
+ * need none where it cannot be had.  The synchronous
  * host-pointer calls use their own buffers.  No reference counterpart (the
  * reference has no device workspace). */
 /* Grows each of the context's device workspaces to at least `bytes`. */

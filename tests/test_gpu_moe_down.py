@@ -10,7 +10,7 @@ from tests.test_gpu_moe_stages import check_stages, ctx, run_layer  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(1, 512, 256, 8, 4), (4, 512, 256, 8, 4), (2, 1280, 512, 16, 6), (1, 256, 1024, 4, 2), (1, 256, 2048, 3, 2),
+CASES = [(1, 512, 256, 8, 4), (8, 512, 256, 8, 4), (2, 1280, 512, 16, 6), (1, 256, 1024, 4, 2), (1, 256, 2048, 3, 2),
          (1, 256, 2304, 3, 2), (1, 256, 256, 40, 33)]  # T, H, F, E, k
 CASES32 = [(1, 288, 32, 8, 4), (3, 544, 288, 8, 4), (2, 256, 1056, 4, 2)]
 
