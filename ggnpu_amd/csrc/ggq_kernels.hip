@@ -4346,14 +4346,15 @@ __global__ __launch_bounds__(1024) void moe_group_small_kernel(const int32_t* __
     // Wavefront w ranks the pairs of its slice [w * S, (w + 1) * S), 64 at
     // a time: lanes holding the same expert are found with one ballot per
     // bit of the expert id; a pair's rank is its count of such lanes below
-    // it plus the slice's earlier pairs of that expert.  The rank goes to
-    // pos_of (read back by the same lane below).
+    // it plus the slice's earlier pairs of that expert.  Experts and ranks of
+    // up to 4096 pairs stay in registers (512 tokens, top 8: the layer 232.2 ->
+    // 229.6 us; one and 64 tokens the same); beyond, the ranks go to pos_of, read
+    // back by the same lane below.
     const int S = ((n + 16 * 64 - 1) / (16 * 64)) * 64;
     const uint64_t below = (1ull << lane) - 1ull;
-    for (int f0 = wave * S; f0 < (wave + 1) * S && f0 < n; f0 += 64) {
-        const int f = f0 + lane;
-        const bool ok = f < n;
-        const int e = ok ? expert_id(sel[f], E) : 0;
+    constexpr int kHeld = 4;
+    int held_e[kHeld], held_r[kHeld];
+    auto rank_of = [&](bool ok, int e) -> int {
         uint64_t same = __ballot(ok);
 #pragma unroll
         for (int bit = 0; bit < 8; bit++) {
@@ -4362,7 +4363,22 @@ __global__ __launch_bounds__(1024) void moe_group_small_kernel(const int32_t* __
         }
         const int before = hist[wave][e];
         if (ok && (same & below) == 0) hist[wave][e] = before + __popcll(same);  // the first such lane
-        if (ok) pos_of[f] = before + __popcll(same & below);
+        return before + __popcll(same & below);
+    };
+    if (S <= 64 * kHeld) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++) {
+            const int f = wave * S + 64 * i + lane;
+            if (64 * i >= S || wave * S + 64 * i >= n) break;
+            held_e[i] = f < n ? expert_id(sel[f], E) : 0;
+            held_r[i] = rank_of(f < n, held_e[i]);
+        }
+    } else {
+        for (int f0 = wave * S; f0 < (wave + 1) * S && f0 < n; f0 += 64) {
+            const int f = f0 + lane;
+            const int r = rank_of(f < n, f < n ? expert_id(sel[f], E) : 0);
+            if (f < n) pos_of[f] = r;
+        }
     }
     __syncthreads();
     // Expert totals, their exclusive scan (four wavefronts cover 256
@@ -4396,14 +4412,19 @@ __global__ __launch_bounds__(1024) void moe_group_small_kernel(const int32_t* __
         start[tid] = b0;  // the end of expert tid's rows
     }
     __syncthreads();
-    for (int f0 = wave * S; f0 < (wave + 1) * S && f0 < n; f0 += 64) {
-        const int f = f0 + lane;
-        if (f < n) {
-            const int e = expert_id(sel[f], E);
-            const int pos = hist[wave][e] + pos_of[f];
-            tok_idx[pos] = f / topk;
-            pos_of[f] = pos;
+    auto place = [&](int f, int e, int r) {
+        const int pos = hist[wave][e] + r;
+        tok_idx[pos] = f / topk;
+        pos_of[f] = pos;
+    };
+    if (S <= 64 * kHeld) {
+#pragma unroll
+        for (int i = 0; i < kHeld; i++) {
+            const int f = wave * S + 64 * i + lane;
+            if (64 * i < S && f < n) place(f, held_e[i], held_r[i]);
         }
+    } else {
+        for (int f = wave * S + lane; f < (wave + 1) * S && f < n; f += 64) place(f, expert_id(sel[f], E), pos_of[f]);
     }
     // The shared expert's group end and token rows, and the grouped int8
     // launches' chunk lists from the offsets just written, saving their own
