@@ -19,7 +19,8 @@ LIB = os.path.join(LIB_DIR, "libggq_hip.so")
 # it calls the entry point through a pointer the caller passes)
 HOST_BENCH = os.path.join(LIB_DIR, "libggq_host_bench.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
-SOURCES = ["ggq_kernels.hip", "ggq_gemv_i8.hip", "ggq_gemm_f16.hip", "ggq_gemm_rows.hip", "ggq_api.cpp", "ggq_encode.cpp", "ggq_gguf.cpp"]
+SOURCES = ["ggq_kernels.hip", "ggq_gemv_i8.hip", "ggq_gemm_f16.hip", "ggq_gemm_rows.hip", "ggq_moe_down.hip",
+           "ggq_api.cpp", "ggq_encode.cpp", "ggq_gguf.cpp"]
 CXX = os.environ.get("CXX", "g++")
 # Host-only sources go through the host compiler against the HIP runtime API.
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",

@@ -546,6 +546,37 @@ __device__ __forceinline__ int8_t to_i8(float v) {
     return (int8_t)(int)r;
 }
 
+// Sum over aligned groups of 2^lg lanes (lg = 0..6): afterwards every lane of
+// a group of <= 32 lanes holds the group sum; for lg = 6 lane 0 holds the
+// wavefront sum.
+template <int CTRL> __device__ __forceinline__ float dpp_addc(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float group_sum(float v, int lg) {
+    if (lg >= 1) v = dpp_addc<0xB1>(v);   // quad_perm [1,0,3,2]: xor 1
+    if (lg >= 2) v = dpp_addc<0x4E>(v);   // quad_perm [2,3,0,1]: xor 2
+    if (lg >= 3) v = dpp_addc<0x141>(v);  // row_half_mirror: the other quad of 8
+    if (lg >= 4) v = dpp_addc<0x140>(v);  // row_mirror: the other half of 16
+    if (lg >= 5) v += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));  // xor 16
+    if (lg >= 6) v += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
+    return v;
+}
+
+// ------------------------------------------------------------- MoE -----
+// Selections come from moe_route_kernel and are below E; the clamp keeps the
+// LDS histograms and the output positions in range regardless.
+__device__ __forceinline__ int expert_id(int e, int E) { return e < 0 ? 0 : e >= E ? E - 1 : e; }
+
+// The caller's copies of token t's experts and weights, written by the token's
+// first workgroup (top_k <= 64 of its threads): no copies of their own behind
+// the layer (two of them cost 2.8 us after one token, 9.6 after 64).
+__device__ __forceinline__ void pick_out(const MoePick& p, const float* wsel, int t, int topk) {
+    if (blockIdx.x || (int)threadIdx.x >= topk) return;
+    const int at = t * topk + threadIdx.x;
+    if (p.sel_out) p.sel_out[at] = p.sel[at];
+    if (p.w_out) p.w_out[at] = wsel[at];
+}
+
 // ------------------------------------------------- MoE chunk lists -----
 // (group, first row) chunk lists for grouped launches (struct ChunkList,
 // ggq_launch.h).
