@@ -55,9 +55,20 @@ struct Work {
 struct Lane {
     hipStream_t stream = nullptr;
     Buffer b;
-    unsigned long long capture = 0;  // the capture whose graph holds the buffer's address (0: none)
 };
-constexpr size_t kMaxLanes = 8, kMaxCapturedLanes = 16;
+constexpr size_t kMaxLanes = 8;
+
+// The same for a stream of a graph capture.  Nothing orders the graph's replays
+// with eager calls, those queued before the capture included, so a capture
+// never gets a buffer that an eager call has used: its buffers are cut from
+// memory that eager calls set aside, at most kCaptureBytes of a context, and
+// stay the graph's until ggq_destroy.
+struct CaptureLane {
+    unsigned long long capture;
+    hipStream_t stream;
+    Buffer b;
+};
+constexpr size_t kCaptureBytes = size_t(8) << 30;
 
 }  // namespace
 
@@ -73,7 +84,10 @@ struct ggq_ctx {
     Work host;  // workspace of the synchronous host-pointer entry points (never
                 // shared with device calls that may still run on other streams)
     std::vector<Lane> lanes;     // workspace of the fp16 GEMM on the *_dev entry points
-    size_t captured_lanes = 0;   // lane buffers that captured graphs keep
+    std::vector<CaptureLane> capture_lanes;
+    Buffer aside;                // memory for captures, its first aside_used bytes in use
+    size_t aside_used = 0, aside_total = 0;  // (total: outgrown allocations too)
+    size_t lane_need = 0;        // the largest buffer an eager call asked for
     Buffer io;  // staging of host A / C for the synchronous entry points
     Buffer logits;  // vocab projection output when the caller does not keep it
     Buffer attn;  // attention chunk partials
@@ -133,12 +147,51 @@ int grow(ggq_ctx* c, Buffer& b, size_t need, hipStream_t s, const char* what) {
     return GGQ_OK;
 }
 
+inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Device memory while another thread may have a capture running (relaxed: the
+// allocation is no part of it).  Null when there is none.
+void* alloc_beside_captures(size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipThreadExchangeStreamCaptureMode(&mode);
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, bytes);
+    hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+// At least `bytes` set aside for captures, where the bound allows.
+void set_aside(ggq_ctx* c, size_t bytes) {
+    if (c->aside.size - c->aside_used >= bytes) return;
+    const size_t sz = 2 * align256(bytes);
+    if (sz > kCaptureBytes - c->aside_total) return;
+    void* p = alloc_beside_captures(sz);
+    if (!p) return;
+    if (c->aside.ptr) c->retired.push_back(c->aside.ptr);
+    c->aside = Buffer{p, sz};
+    c->aside_used = 0;
+    c->aside_total += sz;
+}
+
+void* capture_lane(ggq_ctx* c, hipStream_t s, unsigned long long id, size_t bytes) {
+    for (const CaptureLane& l : c->capture_lanes)
+        if (l.capture == id && l.stream == s && l.b.size >= bytes) return l.b.ptr;
+    // one buffer for the largest call where that is left
+    const size_t left = c->aside.size - c->aside_used, most = align256(std::max(bytes, c->lane_need));
+    const size_t sz = most <= left ? most : align256(bytes);
+    if (sz > left) return nullptr;
+    const Buffer b{(char*)c->aside.ptr + c->aside_used, sz};
+    c->capture_lanes.push_back(CaptureLane{id, s, b});
+    c->aside_used += sz;
+    return b.ptr;
+}
+
 // `bytes` of the stream's lane, or null when it cannot have them now (the
 // caller then takes a path without this workspace): more streams than lanes,
-// no memory, hipStreamPerThread (one handle for several streams), or a
-// capture that would have to allocate.  A buffer that a captured graph uses
-// is left to that graph: later calls on the stream get another one, so a
-// replay on some other stream never meets them.
+// no memory, hipStreamPerThread (one handle for several streams), or a capture
+// for which not enough was set aside.
 void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
     if (s == hipStreamPerThread) return nullptr;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -147,45 +200,28 @@ void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
         (void)hipGetLastError();
         return nullptr;
     }
+    if (cs != hipStreamCaptureStatusNone)
+        return cs == hipStreamCaptureStatusActive ? capture_lane(c, s, id, bytes) : nullptr;
+    c->lane_need = std::max(c->lane_need, bytes);
+    set_aside(c, c->lane_need);
     Lane* l = nullptr;
     for (Lane& x : c->lanes)
         if (x.stream == s) l = &x;
-    if (cs != hipStreamCaptureStatusNone) {
-        if (cs != hipStreamCaptureStatusActive || !l || l->b.size < bytes) return nullptr;
-        if (l->capture != id) {
-            if (l->capture || c->captured_lanes >= kMaxCapturedLanes) return nullptr;
-            l->capture = id;
-            c->captured_lanes++;
-        }
-        return l->b.ptr;
-    }
     if (!l) {
         if (c->lanes.size() >= kMaxLanes) return nullptr;
         c->lanes.emplace_back();
         l = &c->lanes.back();
         l->stream = s;
     }
-    if (l->capture || l->b.size < bytes) {
-        // relaxed: the allocation is no part of a capture another thread may
-        // have running
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        hipThreadExchangeStreamCaptureMode(&mode);
-        void* p = nullptr;
-        const size_t sz = l->capture ? std::max(bytes, l->b.size) : std::max(bytes, 2 * l->b.size);
-        const hipError_t e = hipMalloc(&p, sz);
-        hipThreadExchangeStreamCaptureMode(&mode);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+    if (l->b.size < bytes) {
+        const size_t sz = std::max(bytes, 2 * l->b.size);
+        void* p = alloc_beside_captures(sz);
+        if (!p) return nullptr;
         if (l->b.ptr) c->retired.push_back(l->b.ptr);
         l->b = Buffer{p, sz};
-        l->capture = 0;
     }
     return l->b.ptr;
 }
-
-inline size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Where a call's scratch memory comes from: the growable buffers of a Work,
 // or one fixed region (activation workspace first, split-K partials after).
@@ -721,6 +757,7 @@ void ggq_destroy(ggq_ctx* c) {
     for (void* p : c->retired) hipFree(p);
     for (Lane& l : c->lanes)
         if (l.b.ptr) hipFree(l.b.ptr);
+    if (c->aside.ptr) hipFree(c->aside.ptr);
     if (c->io.ptr) hipFree(c->io.ptr);
     if (c->logits.ptr) hipFree(c->logits.ptr);
     if (c->attn.ptr) hipFree(c->attn.ptr);

@@ -10,7 +10,7 @@ import pytest
 
 import ggnpu_amd.lib as gl
 from tests import test_gpu_parity as t
-from tests.gpu_util import dev
+from tests.gpu_util import dev, host
 
 pytestmark = pytest.mark.gpu
 
@@ -123,5 +123,60 @@ def test_capture_needs_no_workspace_on_the_panel_gemm(orc):
             g.replay()
             torch.cuda.synchronize()
             assert orc.rel_l2(y.cpu().numpy(), orc.mul_mat_f64(8, raw, N, K, A, 1)) < t.TOL
+    finally:
+        c.close()
+
+
+def capture(g, s, work):
+    """torch.cuda.graph without its synchronizations: work queued on `s` may still run."""
+    import torch
+    with torch.cuda.stream(s):
+        g.capture_begin()
+        work()
+        g.capture_end()
+
+
+def f32_call(c, t_, W, N, K, x, y, M, s):
+    c.check(c.lib.ggq_mul_mat_dev(c.h, ctypes.c_void_p(W.data_ptr()), t_, N, K, ctypes.c_void_p(x.data_ptr()), K,
+                                  ctypes.c_void_p(y.data_ptr()), N, M, 0, ctypes.c_void_p(s.cuda_stream)), "mul_mat")
+
+
+@pytest.mark.parametrize("N,K,M", [(2064, 2048, 40), (2064, 4352, 16)])
+def test_capture_beside_queued_eager_calls(orc, N, K, M):
+    """fp32 many-row calls (planes; the slices' sums of few rows) queued on a
+    stream before a capture on it still run while the graph replays on another
+    stream: neither disturbs the other, bit for bit."""
+    import torch
+    c = gl.Context(0)
+    try:
+        raw = t.weights(14, N, K, seed=6)
+        W = dev(raw)
+        x = [torch.randn((M, K), device="cuda") for _ in range(2)]
+        y = [torch.zeros((M, N), device="cuda") for _ in range(17)]
+        s, other = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        want = []
+        for a in x:
+            f32_call(c, 14, W, N, K, a, y[0], M, s)
+            torch.cuda.synchronize()
+            want.append(y[0].clone())
+        assert orc.rel_l2(host(want[0])[:, :64], orc.mul_mat_f64(14, raw[: 64 * (K // 256) * 210], 64, K, host(x[0]), 0)) < t.TOL
+        for _ in range(3):
+            for v in y:
+                v.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                torch.cuda._sleep(5_000_000)
+            for i in range(16):
+                f32_call(c, 14, W, N, K, x[0], y[i], M, s)
+            g = torch.cuda.CUDAGraph()
+            capture(g, s, lambda: [f32_call(c, 14, W, N, K, x[1], y[16], M, s) for _ in range(16)])
+            with torch.cuda.stream(other):
+                for _ in range(8):
+                    g.replay()
+            torch.cuda.synchronize()
+            for i in range(16):
+                assert torch.equal(y[i], want[0]), i
+            assert torch.equal(y[16], want[1])
     finally:
         c.close()
