@@ -12,6 +12,7 @@
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -299,6 +300,13 @@ struct GemmEntry {
 constexpr int kGemmMinRows = 9;
 enum { GEMM_F32 = 0, GEMM_Q8_ROW = 1, GEMM_CODES = 2 };
 
+// GGQ_GEMV_MFMA=0: fp32 rows stay on the FMA kernels, where a row's result
+// does not depend on the rows beside it.
+bool fma_only() {
+    const char* e = getenv("GGQ_GEMV_MFMA");
+    return e && *e && atoi(e) == 0;
+}
+
 // Whether M rows against `cols` columns of one type run on the fp16 GEMM
 // (times in us, earlier kernels -> fp16 GEMM).
 //   fp32 rows: the decode GEMVs' passes of four rows are cheaper for small
@@ -316,6 +324,7 @@ bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
     const bool blocks32 = type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL;
     const int64_t w = cols * K, work = w * M;
     if (mode == GEMM_F32) {
+        if (fma_only()) return false;
         // (the wavefronts of few columns take long K in turn: 333 x 16384 Q4_K,
         // 48 rows 36 -> 71, Q8_0, 64 rows 49 -> 84)
         if (blocks32) return M >= 48 && cols * M >= 49152 && work >= (int64_t)256 << 20;
@@ -356,7 +365,7 @@ struct GroupShape {
 //   16, 8208 x 1536 16 -> 13, 18 -> 13, 36 -> 17.
 constexpr int kRowsMin = 5;
 bool gemm_rows_takes(const GroupShape& g, int K, int M) {
-    if (M < kRowsMin || M > 32) return false;
+    if (M < kRowsMin || M > 32 || fma_only()) return false;
     const int64_t w = g.cols * K, mi = 1 << 20;
     const bool mixed = g.n_types() > 1;
     if (g.types & (1u << GGQ_TYPE_Q8_0 | 1u << GGQ_TYPE_IQ4_NL)) {

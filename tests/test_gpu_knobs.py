@@ -67,6 +67,22 @@ def test_fma_path_batch_invariant(ctx, orc, knob, ty):
             assert np.array_equal(batch[m].view(np.uint32), alone[0].view(np.uint32)), (M, m)
 
 
+@pytest.mark.parametrize("knob", [("GGQ_GEMV_MFMA", "0")], indirect=True)
+@pytest.mark.parametrize("ty,M,act", [(12, 8, 0), (14, 12, 0), (12, 40, 0), (20, 48, 2), (13, 32, 2)])
+def test_fma_path_batch_invariant_many_rows(ctx, orc, knob, ty, M, act):
+    """The same where the default routing multiplies the rows on the fp16 matrix
+    cores: 5 to 32 rows resident in registers, many rows from planes."""
+    import numpy as np
+    K, N = 2048, 4112
+    raw = np.tile(t.weights(ty, 257, K, seed=ty), 16)
+    A = np.random.default_rng(ty).standard_normal((M, K)).astype(np.float32)
+    batch = t.run_mm(ctx, ty, raw, N, K, A, act)
+    assert np.isfinite(batch).all()
+    for m in (0, 3, M - 1):
+        alone = t.run_mm(ctx, ty, raw, N, K, A[m:m + 1], act)
+        assert np.array_equal(batch[m].view(np.uint32), alone[0].view(np.uint32)), m
+
+
 @pytest.mark.parametrize("knob", [("GGQ_I8_MIN_BYTES", "0")], indirect=True)
 @pytest.mark.parametrize("name", ["Q4_K", "Q6_K", "Q8_0", "IQ4_XS"])
 def test_i8_gemv_all_sizes(ctx, orc, knob, name):
