@@ -163,11 +163,14 @@ void* alloc_beside_captures(size_t bytes) {
     return nullptr;
 }
 
-// At least `bytes` set aside for captures, where the bound allows.
-void set_aside(ggq_ctx* c, size_t bytes) {
-    if (c->aside.size - c->aside_used >= bytes) return;
-    const size_t sz = 2 * align256(bytes);
-    if (sz > kCaptureBytes - c->aside_total) return;
+// At least `bytes` set aside for captures, where the bound allows; `copies` of
+// them when that takes new memory.
+void set_aside(ggq_ctx* c, size_t bytes, size_t copies) {
+    if (c->aside.size - c->aside_used >= bytes || !bytes) return;
+    bytes = align256(bytes);
+    copies = std::min(copies, (kCaptureBytes - c->aside_total) / bytes);
+    if (!copies) return;
+    const size_t sz = copies * bytes;
     void* p = alloc_beside_captures(sz);
     if (!p) return;
     if (c->aside.ptr) c->retired.push_back(c->aside.ptr);
@@ -203,8 +206,9 @@ void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
     }
     if (cs != hipStreamCaptureStatusNone)
         return cs == hipStreamCaptureStatusActive ? capture_lane(c, s, id, bytes) : nullptr;
+    // for eight captures in a row, two where that would be more than 256 MB
     c->lane_need = std::max(c->lane_need, bytes);
-    set_aside(c, c->lane_need);
+    set_aside(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
     Lane* l = nullptr;
     for (Lane& x : c->lanes)
         if (x.stream == s) l = &x;
@@ -412,11 +416,36 @@ int gemm_rows_per_pass(int K, int M, bool codes) {
     return (size_t)M <= rows ? M : (int)std::max<size_t>(rows, 128);
 }
 
+// Workspace of the int8 GEMM for per-row int8 rows: codes and scales.
+size_t q8_rows_bytes(int K, int M) { return align256((size_t)M * K) + align256(sizeof(float) * (size_t)M * (K / 32)); }
+
+// The workspace that int8 rows need without planes.  Eager calls keep it sized
+// though they do not use it, so that a capture after them that finds no planes
+// left records the int8 GEMMs and is not refused.
+void size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M) {
+    size_t ws_bytes = 0, part_bytes = 0;
+    int Ns[GGQ_MAX_BATCH];
+    bool one_type = true;
+    for (int i = 0; i < n; i++) {
+        Ns[i] = d[i].N;
+        one_type = one_type && d[i].type == d[0].type;
+        if (ggq::gemm_panel_eligible(d[i].type, K, M, A, lda)) continue;
+        part_bytes = std::max(part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[i].type, &Ns[i], 1, K, M)));
+        if (mode == GEMM_Q8_ROW) ws_bytes = q8_rows_bytes(K, M);
+    }
+    if (part_bytes && one_type && n > 1 && n <= GGQ_MAX_GEMM_BATCH)
+        part_bytes = std::max(part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[0].type, Ns, n, K, M)));
+    void* ws;
+    float* part;
+    if (ar.get(ws_bytes, part_bytes, &ws, &part, "workspace") != GGQ_OK) (void)hipGetLastError();
+}
+
 // True when the call was taken (*st its status); false: not queued.
 bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n, int K, int mode, const float* A,
               int lda, const int8_t* qa, const float* sa, int M, hipStream_t s, int* st) {
     const bool codes = mode != GEMM_F32;
     const int step = gemm_rows_per_pass(K, M, codes);
+    if (codes && ar.w == &c->dev) size_int8_gemm(c, ar, d, n, K, mode, A, lda, M);
     void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
     if (!ws) return false;
     hipError_t e;
@@ -907,6 +936,7 @@ int ggq_reserve(ggq_ctx* c, int64_t bytes) {
     int st;
     for (Buffer* buf : {&c->dev.ws, &c->dev.part, &c->logits, &c->attn})
         if ((st = grow(c, *buf, b, c->stream, "reserve")) != GGQ_OK) return st;
+    set_aside(c, b, 1);
     return set_status(c, GGQ_OK);
     GGQ_END(c)
 }

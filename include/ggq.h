@@ -85,12 +85,18 @@ int ggq_sync(ggq_ctx* ctx);
  * made while its stream is being captured never allocates: if its workspace
  * is too small it fails with GGQ_ERROR and says so in
  * ggq_last_error_message.  Size the workspace before a capture by running
- * the captured calls once outside it, or with ggq_reserve.  Matmuls of 5 rows
- * and more also use a buffer per stream (at most 8 streams), and kernels that
- * need none where it cannot be had.  The synchronous
+ * the captured calls once outside it, or with ggq_reserve.
+ * Matmuls of 5 rows and more also use a buffer per stream (at most 8 streams),
+ * and other kernels where it cannot be had: the same products, rounded in
+ * another order, in several times the time.  Each capture gets a buffer of its
+ * own that stays with its graph: a call outside a capture, on any stream, sets
+ * aside what eight captures of the largest such call so far need (two where
+ * that is more than 256 MB), ggq_reserve its bytes, at most 8 GiB of a context.
+ * Run a call between captures when there are more of them.  The synchronous
  * host-pointer calls use their own buffers.  No reference counterpart (the
  * reference has no device workspace). */
-/* Grows each of the context's device workspaces to at least `bytes`. */
+/* Grows each of the context's device workspaces, and what is set aside for
+ * captures, to at least `bytes`. */
 int ggq_reserve(ggq_ctx* ctx, int64_t bytes);
 
 /* ------------------------------------------------ host-pointer, synchronous */

@@ -10,7 +10,7 @@ import pytest
 
 import ggnpu_amd.lib as gl
 from tests import test_gpu_parity as t
-from tests.gpu_util import dev, host
+from tests.gpu_util import dev, host, ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -178,5 +178,79 @@ def test_capture_beside_queued_eager_calls(orc, N, K, M):
             for i in range(16):
                 assert torch.equal(y[i], want[0]), i
             assert torch.equal(y[16], want[1])
+    finally:
+        c.close()
+
+
+# (type, M, K): Q6_K rows and long rows of Q4_K use the int8 GEMM's workspace without planes
+@pytest.mark.parametrize("entry", ["row", "codes", "batch"])
+@pytest.mark.parametrize("ty,M,K", [(14, 40, 2048), (12, 16, 4352)])
+def test_one_warm_up_prepares_every_capture(orc, ty, M, K, entry):
+    """int8 rows: after one eager call, any number of captures on another stream
+    are accepted; those with planes equal the eager call bit for bit, the ones
+    beyond what was set aside agree with the oracle."""
+    import torch
+    N, captures = 528, 12
+    c = gl.Context(0)
+    try:
+        raw = t.weights(ty, N, K, seed=ty)
+        W = dev(raw)
+        a = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+        x, y = torch.from_numpy(a).cuda(), torch.zeros((M, N), device="cuda")
+        q, sa = torch.zeros((M, K), dtype=torch.int8, device="cuda"), torch.zeros(M, device="cuda")
+        c.check(c.lib.ggq_quantize_act_dev(c.h, ptr(x), K, M, K, 1, ptr(q), ptr(sa), None), "quantize")
+        d = (gl.GemvDesc * 1)()
+        d[0].W, d[0].type, d[0].N, d[0].K, d[0].A, d[0].C = W.data_ptr(), ty, N, K, x.data_ptr(), y.data_ptr()
+
+        def call(s):
+            h = ctypes.c_void_p(s.cuda_stream)
+            if entry == "row":
+                return c.lib.ggq_mul_mat_dev(c.h, ptr(W), ty, N, K, ptr(x), K, ptr(y), N, M, 1, h)
+            if entry == "codes":
+                return c.lib.ggq_mul_mat_q8_dev(c.h, ptr(W), ty, N, K, ptr(q), ptr(sa), M, ptr(y), N, h)
+            return c.lib.ggq_mul_mat_batch_act_dev(c.h, d, 1, M, 1, h)
+        warm, s = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        c.check(call(warm), "warm-up")
+        torch.cuda.synchronize()
+        want = y.clone()
+        ref = orc.mul_mat_f64(ty, raw, N, K, a, 1)
+        status, graphs = [], []
+        for _ in range(captures):
+            g = torch.cuda.CUDAGraph()
+            capture(g, s, lambda: status.append(call(s)))
+            graphs.append(g)
+        assert status == [0] * captures
+        for i, g in enumerate(graphs):
+            for _ in range(2):
+                y.zero_()
+                g.replay()
+                torch.cuda.synchronize()
+                assert orc.rel_l2(host(y), ref) < t.TOL
+                if i < 8:
+                    assert torch.equal(y, want), i
+    finally:
+        c.close()
+
+
+def test_reserve_prepares_captures_of_many_rows(orc):
+    """After ggq_reserve alone a capture records what an eager call runs."""
+    import torch
+    N, K, M = 2064, 2048, 40
+    c = gl.Context(0)
+    try:
+        W = dev(t.weights(14, N, K, seed=1))
+        x, y, want = torch.randn((M, K), device="cuda"), torch.zeros((M, N), device="cuda"), torch.zeros((M, N), device="cuda")
+        s = torch.cuda.Stream()
+        c.check(c.lib.ggq_reserve(c.h, 4 << 20), "reserve")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        capture(g, s, lambda: f32_call(c, 14, W, N, K, x, y, M, s))
+        f32_call(c, 14, W, N, K, x, want, M, s)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
     finally:
         c.close()
