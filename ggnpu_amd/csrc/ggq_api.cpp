@@ -51,13 +51,22 @@ struct Work {
 // Planes of the activation rows of the fp16 GEMM, one buffer per stream: the
 // calls that take that GEMM also run at sizes and activation treatments that
 // need no other workspace, and callers may queue those on several streams at
-// once.  At most kMaxLanes streams of a context have one; calls on further
-// streams take the kernels that need none.
+// once.
 struct Lane {
     hipStream_t stream = nullptr;
     Buffer b;
 };
 constexpr size_t kMaxLanes = 8;
+
+// Buffers that all further streams share (a context keeps no count of streams
+// that are gone): a call waits, on its stream, for the event behind the
+// buffer's last use.
+struct SharedLane {
+    hipStream_t stream = nullptr;  // of the last use; a hint only
+    Buffer b;
+    hipEvent_t ev = nullptr;
+};
+constexpr size_t kSharedLanes = 8;
 
 // The same for a stream of a graph capture.  Nothing orders the graph's replays
 // with eager calls, those queued before the capture included, so a capture
@@ -85,6 +94,9 @@ struct ggq_ctx {
     Work host;  // workspace of the synchronous host-pointer entry points (never
                 // shared with device calls that may still run on other streams)
     std::vector<Lane> lanes;     // workspace of the fp16 GEMM on the *_dev entry points
+    SharedLane shared[kSharedLanes];
+    size_t shared_next = 0;
+    SharedLane* leased = nullptr;  // the shared lane of the call being queued
     std::vector<CaptureLane> capture_lanes;
     Buffer aside;                // memory for captures, its first aside_used bytes in use
     size_t aside_used = 0, aside_total = 0;  // (total: outgrown allocations too)
@@ -192,12 +204,48 @@ void* capture_lane(ggq_ctx* c, hipStream_t s, unsigned long long id, size_t byte
     return b.ptr;
 }
 
-// `bytes` of the stream's lane, or null when it cannot have them now (the
-// caller then takes a path without this workspace): more streams than lanes,
-// no memory, hipStreamPerThread (one handle for several streams), or a capture
-// for which not enough was set aside.
+// `b` of at least `bytes`; the outgrown allocation stays for work queued on it.
+bool grow_lane(ggq_ctx* c, Buffer& b, size_t bytes) {
+    if (b.size >= bytes) return true;
+    const size_t sz = std::max(bytes, 2 * b.size);
+    void* p = alloc_beside_captures(sz);
+    if (!p) return false;
+    if (b.ptr) c->retired.push_back(b.ptr);
+    b = Buffer{p, sz};
+    return true;
+}
+
+// A shared lane for the call being queued on `s`; lane_done ends its use.
+void* shared_lane(ggq_ctx* c, hipStream_t s, size_t bytes) {
+    SharedLane* l = nullptr;
+    for (SharedLane& x : c->shared)
+        if (x.ev && x.stream == s) l = &x;
+    if (!l) l = &c->shared[c->shared_next++ % kSharedLanes];
+    hipError_t e = hipSuccess;
+    if (l->ev) e = hipStreamWaitEvent(s, l->ev, 0);
+    else if ((e = hipEventCreateWithFlags(&l->ev, hipEventDisableTiming)) != hipSuccess) l->ev = nullptr;
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e != hipSuccess || !grow_lane(c, l->b, bytes)) return nullptr;
+    l->stream = s;
+    c->leased = l;
+    return l->b.ptr;
+}
+
+// The call's work on `s` is queued.
+void lane_done(ggq_ctx* c, hipStream_t s) {
+    if (!c->leased) return;
+    if (hipEventRecord(c->leased->ev, s) != hipSuccess) {
+        (void)hipGetLastError();
+        hipStreamSynchronize(s);
+    }
+    c->leased = nullptr;
+}
+
+// `bytes` for the rows of a call on `s`, or null when there are none now (the
+// caller then takes a path without this workspace): no memory, or a capture for
+// which not enough was set aside or whose stream cannot be told from others
+// (hipStreamPerThread: one handle for several).
 void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
-    if (s == hipStreamPerThread) return nullptr;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(s, &cs, &id) != hipSuccess) {
@@ -205,27 +253,21 @@ void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
         return nullptr;
     }
     if (cs != hipStreamCaptureStatusNone)
-        return cs == hipStreamCaptureStatusActive ? capture_lane(c, s, id, bytes) : nullptr;
+        return cs == hipStreamCaptureStatusActive && s != hipStreamPerThread ? capture_lane(c, s, id, bytes) : nullptr;
     // for eight captures in a row, two where that would be more than 256 MB
     c->lane_need = std::max(c->lane_need, bytes);
     set_aside(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
+    if (s == hipStreamPerThread) return shared_lane(c, s, bytes);
     Lane* l = nullptr;
     for (Lane& x : c->lanes)
         if (x.stream == s) l = &x;
     if (!l) {
-        if (c->lanes.size() >= kMaxLanes) return nullptr;
+        if (c->lanes.size() >= kMaxLanes) return shared_lane(c, s, bytes);
         c->lanes.emplace_back();
         l = &c->lanes.back();
         l->stream = s;
     }
-    if (l->b.size < bytes) {
-        const size_t sz = std::max(bytes, 2 * l->b.size);
-        void* p = alloc_beside_captures(sz);
-        if (!p) return nullptr;
-        if (l->b.ptr) c->retired.push_back(l->b.ptr);
-        l->b = Buffer{p, sz};
-    }
-    return l->b.ptr;
+    return grow_lane(c, l->b, bytes) ? l->b.ptr : nullptr;
 }
 
 // Where a call's scratch memory comes from: the growable buffers of a Work,
@@ -257,13 +299,15 @@ struct Arena {
         return GGQ_OK;
     }
     // Planes of the fp16 GEMM beside `ws_bytes` taken with get(), or null
-    // when the call should run without them.
+    // when the call should run without them; planes_done once the work that
+    // uses them is queued.
     void* planes(size_t ws_bytes, size_t bytes) {
         if (w == &c->dev) return lane_ws(c, s, bytes);
         if (w) return grow(c, w->part, bytes, s, "workspace") == GGQ_OK ? w->part.ptr : nullptr;
         const size_t off = align256(ws_bytes);
         return off + bytes <= cap ? fixed + off : nullptr;
     }
+    void planes_done() { lane_done(c, s); }
 };
 
 Arena dev_arena(ggq_ctx* c, hipStream_t s) { return Arena{c, &c->dev, nullptr, 0, s}; }
@@ -405,7 +449,9 @@ bool gemm_rows(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n
         gd[i] = ggq::GemmDesc{d[i].W, d[i].C, d[i].N, d[i].ldc};
         types[i] = d[i].type;
     }
-    *st = hip_status(c, ggq::launch_gemm_rows(gd, types, n, K, A, lda, M, ws, s), "gemm_rows");
+    const hipError_t e = ggq::launch_gemm_rows(gd, types, n, K, A, lda, M, ws, s);
+    ar.planes_done();
+    *st = hip_status(c, e, "gemm_rows");
     return true;
 }
 
@@ -448,14 +494,13 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
     if (codes && ar.w == &c->dev) size_int8_gemm(c, ar, d, n, K, mode, A, lda, M);
     void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
     if (!ws) return false;
-    hipError_t e;
-    for (int m0 = 0; m0 < M; m0 += step) {
+    hipError_t e = hipSuccess;
+    for (int m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
         const int rows = std::min(step, M - m0);
         e = ggq::launch_gemm_f16_prep(mode, A ? A + (size_t)m0 * lda : nullptr, lda, qa ? qa + (size_t)m0 * K : nullptr,
                                       K, rows, ws, s);
-        if (e != hipSuccess) return *st = hip_status(c, e, "gemm_f16 rows"), true;
         bool done[GGQ_MAX_BATCH] = {};
-        for (int i = 0; i < n; i++) {
+        for (int i = 0; i < n && e == hipSuccess; i++) {
             if (done[i]) continue;
             ggq::GemmDesc gd[GGQ_MAX_GEMM_BATCH];
             int ng = 0;
@@ -465,10 +510,11 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
                     done[j] = true;
                 }
             e = ggq::launch_gemm_f16(d[i].type, gd, ng, K, rows, codes, sa ? sa + m0 : nullptr, ws, s);
-            if (e != hipSuccess) return *st = hip_status(c, e, "gemm_f16"), true;
         }
     }
-    return *st = set_status(c, GGQ_OK), true;
+    ar.planes_done();
+    *st = hip_status(c, e, "gemm_f16");
+    return true;
 }
 
 // The entries of a batch on the fp16 GEMM, those that share their activations
@@ -795,6 +841,10 @@ void ggq_destroy(ggq_ctx* c) {
     for (void* p : c->retired) hipFree(p);
     for (Lane& l : c->lanes)
         if (l.b.ptr) hipFree(l.b.ptr);
+    for (SharedLane& l : c->shared) {
+        if (l.ev) hipEventDestroy(l.ev);
+        if (l.b.ptr) hipFree(l.b.ptr);
+    }
     if (c->aside.ptr) hipFree(c->aside.ptr);
     if (c->io.ptr) hipFree(c->io.ptr);
     if (c->logits.ptr) hipFree(c->logits.ptr);

@@ -86,9 +86,11 @@ int ggq_sync(ggq_ctx* ctx);
  * is too small it fails with GGQ_ERROR and says so in
  * ggq_last_error_message.  Size the workspace before a capture by running
  * the captured calls once outside it, or with ggq_reserve.
- * Matmuls of 5 rows and more also use a buffer per stream (at most 8 streams),
- * and other kernels where it cannot be had: the same products, rounded in
- * another order, in several times the time.  Each capture gets a buffer of its
+ * Matmuls of 5 rows and more also use a buffer per stream (streams from the
+ * ninth on share eight, and their calls wait for one another where they meet
+ * on one), and other kernels where it cannot be had: the same products, rounded
+ * in another order, in several times the time.  A stream's work is complete
+ * before the stream is destroyed.  Each capture gets a buffer of its
  * own that stays with its graph: a call outside a capture, on any stream, sets
  * aside what eight captures of the largest such call so far need (two where
  * that is more than 256 MB), ggq_reserve its bytes, at most 8 GiB of a context.

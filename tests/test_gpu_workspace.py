@@ -254,3 +254,39 @@ def test_reserve_prepares_captures_of_many_rows(orc):
             assert torch.equal(y, want)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("N,K,M", [(2064, 2048, 40), (2064, 4352, 16)])
+def test_every_stream_runs_the_same_kernels(N, K, M):
+    """Unordered fp32 many-row calls on more streams than a context keeps buffers
+    for, hipStreamPerThread among them, each give the first stream's result bit
+    for bit, also while earlier calls on other streams still run."""
+    import torch
+    c = gl.Context(0)
+    try:
+        W = dev(t.weights(14, N, K, seed=2))
+        streams = [torch.cuda.Stream().cuda_stream for _ in range(20)] + [2]
+        x = [torch.randn((M, K), device="cuda") for _ in streams]
+        y = [torch.zeros((M, N), device="cuda") for _ in streams]
+        want = [torch.zeros((M, N), device="cuda") for _ in streams]
+        torch.cuda.synchronize()
+
+        def call(a, out, s):
+            c.check(c.lib.ggq_mul_mat_dev(c.h, ptr(W), 14, N, K, ptr(a), K, ptr(out), N, M, 0, ctypes.c_void_p(s)), "mul_mat")
+        for a, out in zip(x, want):
+            call(a, out, streams[0])
+        torch.cuda.synchronize()
+        for _ in range(3):
+            for v in y:
+                v.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(torch.cuda.ExternalStream(streams[9])):
+                torch.cuda._sleep(2_000_000)
+            for _ in range(4):
+                for a, out, s in zip(x, y, streams):
+                    call(a, out, s)
+            torch.cuda.synchronize()
+            for i, (out, ref) in enumerate(zip(y, want)):
+                assert torch.equal(out, ref), i
+    finally:
+        c.close()
