@@ -308,6 +308,11 @@ struct Arena {
         return off + bytes <= cap ? fixed + off : nullptr;
     }
     void planes_done() { lane_done(c, s); }
+    // Bytes that planes() can give beside `ws_bytes`, as far as that is fixed.
+    size_t room(size_t ws_bytes) const {
+        if (w) return SIZE_MAX;
+        return cap > align256(ws_bytes) ? cap - align256(ws_bytes) : 0;
+    }
 };
 
 Arena dev_arena(ggq_ctx* c, hipStream_t s) { return Arena{c, &c->dev, nullptr, 0, s}; }
@@ -336,8 +341,8 @@ int check_matmul_shape(ggq_ctx* c, uint32_t type, int64_t N, int64_t K, int M, i
 }
 
 // The matmuls that run on the fp16 GEMM: one activation matrix (fp32 rows A,
-// as they are or quantized per row, or int8 codes qa with row scales sa) and
-// the weights that share it.
+// as they are or quantized per row, or int8 codes qa with scales sa, one a row
+// or one per 32 values) and the weights that share it.
 struct GemmEntry {
     const void* W;
     uint32_t type;
@@ -346,7 +351,7 @@ struct GemmEntry {
     int ldc;
 };
 constexpr int kGemmMinRows = 9;
-enum { GEMM_F32 = 0, GEMM_Q8_ROW = 1, GEMM_CODES = 2 };
+enum { GEMM_F32 = 0, GEMM_Q8_ROW = 1, GEMM_CODES = 2, GEMM_BLOCKS = 3 };  // modes of launch_gemm_f16_prep
 
 // GGQ_GEMV_MFMA=0: fp32 rows stay on the FMA kernels, where a row's result
 // does not depend on the rows beside it.
@@ -440,7 +445,14 @@ bool gemm_rows(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n
     int64_t cols = 0;
     for (int i = 0; i < n; i++) cols += d[i].N;
     if (cols > INT32_MAX) return false;
-    const size_t bytes = ggq::gemm_rows_ws_bytes(K, M, cols);
+    size_t bytes = ggq::gemm_rows_ws_bytes(K, M, cols);
+    // what a fixed region does not hold at once goes in turns of columns (one weight)
+    int64_t turn = cols;
+    if (bytes > ar.room(ws_bytes)) {
+        turn = n == 1 ? (int64_t)(ar.room(ws_bytes) / ggq::gemm_rows_ws_bytes(K, M, 16)) * 16 : 0;
+        if (!turn) return false;
+        bytes = ggq::gemm_rows_ws_bytes(K, M, turn);
+    }
     void* ws = bytes ? ar.planes(ws_bytes, bytes) : nullptr;
     if (bytes && !ws) return false;
     ggq::GemmDesc gd[GGQ_MAX_BATCH];
@@ -449,16 +461,24 @@ bool gemm_rows(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n
         gd[i] = ggq::GemmDesc{d[i].W, d[i].C, d[i].N, d[i].ldc};
         types[i] = d[i].type;
     }
-    const hipError_t e = ggq::launch_gemm_rows(gd, types, n, K, A, lda, M, ws, s);
+    hipError_t e = hipSuccess;
+    if (turn == cols) e = ggq::launch_gemm_rows(gd, types, n, K, A, lda, M, ws, s);
+    else
+        for (int64_t n0 = 0; n0 < cols && e == hipSuccess; n0 += turn) {
+            const ggq::GemmDesc part{(const uint8_t*)d[0].W + n0 * ggq::row_bytes(d[0].type, K), d[0].C + n0,
+                                     (int)std::min(turn, cols - n0), d[0].ldc};
+            e = ggq::launch_gemm_rows(&part, types, 1, K, A, lda, M, ws, s);
+        }
     ar.planes_done();
     *st = hip_status(c, e, "gemm_rows");
     return true;
 }
 
-// Rows per pass over the weights: the planes of a pass stay within 256 MB.
-int gemm_rows_per_pass(int K, int M, bool codes) {
-    const size_t row = ggq::gemm_f16_ws_bytes(K, 128, codes) / 128;
-    const size_t rows = ((size_t(256) << 20) / row) & ~size_t(127);
+// Rows per pass over the weights: the planes of a pass stay within 256 MB and
+// `room` bytes, where 128 rows do.
+int gemm_rows_per_pass(int K, int M, bool codes, size_t room) {
+    const size_t tile = ggq::gemm_f16_ws_bytes(K, 128, codes);
+    const size_t rows = std::min(size_t(256) << 20, room) / tile * 128;
     return (size_t)M <= rows ? M : (int)std::max<size_t>(rows, 128);
 }
 
@@ -467,8 +487,10 @@ size_t q8_rows_bytes(int K, int M) { return align256((size_t)M * K) + align256(s
 
 // The workspace that int8 rows need without planes.  Eager calls keep it sized
 // though they do not use it, so that a capture after them that finds no planes
-// left records the int8 GEMMs and is not refused.
-void size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M) {
+// left records the int8 GEMMs and is not refused.  (A fixed region has to hold
+// it, though the call does without: what its entry point refuses does not
+// depend on the kernel.)
+int size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M) {
     size_t ws_bytes = 0, part_bytes = 0;
     int Ns[GGQ_MAX_BATCH];
     bool one_type = true;
@@ -483,22 +505,24 @@ void size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int
         part_bytes = std::max(part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[0].type, Ns, n, K, M)));
     void* ws;
     float* part;
-    if (ar.get(ws_bytes, part_bytes, &ws, &part, "workspace") != GGQ_OK) (void)hipGetLastError();
+    const int st = ar.get(ws_bytes, part_bytes, &ws, &part, "workspace");
+    if (st != GGQ_OK) (void)hipGetLastError();
+    return st;
 }
 
 // True when the call was taken (*st its status); false: not queued.
 bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n, int K, int mode, const float* A,
               int lda, const int8_t* qa, const float* sa, int M, hipStream_t s, int* st) {
-    const bool codes = mode != GEMM_F32;
-    const int step = gemm_rows_per_pass(K, M, codes);
-    if (codes && ar.w == &c->dev) size_int8_gemm(c, ar, d, n, K, mode, A, lda, M);
+    const bool codes = mode == GEMM_Q8_ROW || mode == GEMM_CODES;
+    const int step = gemm_rows_per_pass(K, M, codes, ar.room(ws_bytes));
+    if (codes && ar.w != &c->host && (*st = size_int8_gemm(c, ar, d, n, K, mode, A, lda, M)) != GGQ_OK && !ar.w) return true;
     void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
     if (!ws) return false;
     hipError_t e = hipSuccess;
     for (int m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
         const int rows = std::min(step, M - m0);
         e = ggq::launch_gemm_f16_prep(mode, A ? A + (size_t)m0 * lda : nullptr, lda, qa ? qa + (size_t)m0 * K : nullptr,
-                                      K, rows, ws, s);
+                                      mode == GEMM_BLOCKS ? sa + (size_t)m0 * (K / 32) : nullptr, K, rows, ws, s);
         bool done[GGQ_MAX_BATCH] = {};
         for (int i = 0; i < n && e == hipSuccess; i++) {
             if (done[i]) continue;
@@ -509,7 +533,7 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
                     gd[ng++] = ggq::GemmDesc{d[j].W, d[j].C + (size_t)m0 * d[j].ldc, d[j].N, d[j].ldc};
                     done[j] = true;
                 }
-            e = ggq::launch_gemm_f16(d[i].type, gd, ng, K, rows, codes, sa ? sa + m0 : nullptr, ws, s);
+            e = ggq::launch_gemm_f16(d[i].type, gd, ng, K, rows, M, codes, mode == GEMM_CODES ? sa + m0 : nullptr, ws, s);
         }
     }
     ar.planes_done();
@@ -634,10 +658,16 @@ int mul_mat_queue(ggq_ctx* c, Arena& ar, const void* W, uint32_t type, int64_t N
             return hip_status(c, e, "quant_act");
         return hip_status(c, ggq::launch_gemm_i8(type, W, (int)N, (int)K, q, sc, M, C, ldc, part, s), "gemm_i8");
     }
+    const bool rows = gemm_rows_takes(type, N, (int)K, M);
+    if (act_mode == GGQ_ACT_Q8_BLOCK32 && !rows && gemm_f16_takes(type, N, (int)K, M, GEMM_F32)) {
+        // the planes come from the codes, so that they have xe's place too in a fixed region
+        if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, q, sc, nullptr, s)) != hipSuccess)
+            return hip_status(c, e, "quant_act");
+        if (gemm_f16(c, ar, x_off, &ge, 1, (int)K, GEMM_BLOCKS, nullptr, 0, q, sc, M, s, &st)) return st;
+    }
     if ((e = ggq::launch_quant_act(A, lda, M, (int)K, act_mode, nullptr, nullptr, xe, s)) != hipSuccess)
         return hip_status(c, e, "quant_act");
-    if (gemm_rows_takes(type, N, (int)K, M) && gemm_rows(c, ar, need, &ge, 1, (int)K, xe, (int)K, M, s, &st)) return st;
-    if (gemm_f16_takes(type, N, (int)K, M, GEMM_F32) && gemm_f16(c, ar, need, &ge, 1, (int)K, GEMM_F32, xe, (int)K, nullptr, nullptr, M, s, &st)) return st;
+    if (rows && gemm_rows(c, ar, need, &ge, 1, (int)K, xe, (int)K, M, s, &st)) return st;
     g.X = xe;
     g.ldx = (int)K;
     return hip_status(c, ggq::launch_gemv(g, s), "gemv");

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
 struct PrepArgs {
     const float* A;
     const int8_t* QA;
-    const float* sa;
+    const float* bs;  // scales of 32 codes, [M][K / 32]
     int lda, M, K, SB, vec;
     h8* XH;
     h8* XL;
@@ -386,7 +386,8 @@ struct PrepArgs {
 constexpr int kPi[8] = {0, 2, 1, 3, 4, 6, 5, 7};
 
 // MODE 0: fp32 rows as hi + lo; 1: fp32 rows quantized per row to int8 codes
-// (the codes and scales of the row quantizer); 2: given int8 codes.
+// (the codes and scales of the row quantizer); 2: given int8 codes; 3: given
+// int8 codes and block scales, whose products are fp32 rows as in 0.
 //
 // Neighbouring lanes hold the same piece of RW neighbouring rows, which lie
 // side by side in the planes (16 RW bytes a run; with a row per workgroup each
@@ -394,13 +395,14 @@ constexpr int kPi[8] = {0, 2, 1, 3, 4, 6, 5, 7};
 // between the row's maximum and the conversion; longer rows are read twice.
 template <int MODE, int RW, int RP, bool VEC>
 __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
+    constexpr bool kCodes = MODE >= 2, kSplit = MODE == 0 || MODE == 3;
     __shared__ float wmax[16 * RW];
     const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
     // a row each: an XCD takes a contiguous range of them, so that their pieces
     // meet in one L2
     const int wg = RW == 1 ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const int m = wg * RW + tid % RW, p0 = tid / RW, ps = blockDim.x / RW, np = a.SB * 32;
-    const int64_t row = (int64_t)(m < a.M ? m : a.M - 1) * (MODE == 2 ? a.K : a.lda);
+    const int64_t row = (int64_t)(m < a.M ? m : a.M - 1) * (kCodes ? a.K : a.lda);
     const size_t tile = (size_t)(m >> 5) * a.SB;
     const int r = m & 31, chunk = ps * RP;
     float v[RP][8];
@@ -411,10 +413,14 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
             const bool in = m < a.M && k < a.K;
             // no branch around the loads: places past the row read its start
             const int64_t at = row + (in ? k : 0);
-            if constexpr (MODE == 2) {
+            if constexpr (kCodes) {
                 const uint2 q = *(const uint2*)(a.QA + at);
+                const float d = MODE == 3 ? a.bs[at >> 5] : 0.0f;
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[i][e] = (float)(int8_t)((e < 4 ? q.x : q.y) >> (8 * (e & 3)));
+                for (int e = 0; e < 8; e++) {
+                    const float x = (float)(int8_t)((e < 4 ? q.x : q.y) >> (8 * (e & 3)));
+                    v[i][e] = MODE == 3 ? __fmul_rn(x, d) : x;
+                }
             } else if (VEC) {
                 const float4 x = *(const float4*)(a.A + at), y = *(const float4*)(a.A + at + 4);
                 v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
@@ -445,7 +451,7 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
         if (lane < RW) wmax[(tid >> 6) * RW + lane] = amax;
         __syncthreads();
         for (int o = 0; o < waves; o++) amax = fmaxf(amax, wmax[o * RW + tid % RW]);
-        if constexpr (MODE == 0) {
+        if constexpr (kSplit) {
             if (amax > 0.0f) {  // the largest magnitude into [2^14, 2^15)
                 int x2;
                 (void)frexpf(amax, &x2);
@@ -469,15 +475,15 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float x = v[i][kPi[e]];
-                const float y = MODE == 0 ? ldexpf(x, ex) : MODE == 1 ? (float)to_i8(__fmul_rn(x, inv)) : x;
+                const float y = kSplit ? ldexpf(x, ex) : MODE == 1 ? (float)to_i8(__fmul_rn(x, inv)) : x;
                 hi[e] = (_Float16)y;
                 lo[e] = (_Float16)(y - (float)hi[e]);
-                gs += MODE == 0 ? (float)hi[e] + (float)lo[e] : y;
+                gs += kSplit ? (float)hi[e] + (float)lo[e] : y;
             }
             const int g = p >> 2, h = (p >> 1) & 1, u = p & 1;
             const size_t at = (tile * 16 + 2 * g + u) * 64 + 32 * h + r;
             a.XH[at] = hi;
-            if constexpr (MODE == 0) a.XL[at] = lo;
+            if constexpr (kSplit) a.XL[at] = lo;
             gs += __shfl_xor(gs, RW, 64);  // the group's four pieces: all of them are in this loop
             gs += __shfl_xor(gs, 2 * RW, 64);
             const float y = gs * 0.03125f;
@@ -506,7 +512,8 @@ void launch_prep_v(const PrepArgs& a, hipStream_t s) {
 }
 template <int MODE>
 void launch_prep(const PrepArgs& a, hipStream_t s) {
-    if (MODE == 2 || a.vec) launch_prep_v<MODE, true>(a, s);
+    if constexpr (MODE >= 2) launch_prep_v<MODE, true>(a, s);
+    else if (a.vec) launch_prep_v<MODE, true>(a, s);
     else launch_prep_v<MODE, false>(a, s);
 }
 
@@ -540,7 +547,7 @@ Planes planes_of(int K, int M, bool two) {
 // bits at K = 8192 2.4e-7, 2.25e-7, 2.15e-7 with one, two, four (the single-
 // row kernels' 2.35e-7).
 template <int T, int AP>
-void launch_t(Args& a, int M, hipStream_t s) {
+void launch_t(Args& a, int M, hipStream_t s) {  // M: the rows of the whole call
     constexpr int kCus = 256;
     // tiles of `cols` x `rows`; returns the grid
     auto tiles = [&](int cols, int rows) {
@@ -549,7 +556,7 @@ void launch_t(Args& a, int M, hipStream_t s) {
             a.p[i].nt0 = a.nt;
             a.nt += (a.p[i].N + cols - 1) / cols;
         }
-        a.mt = (M + rows - 1) / rows;
+        a.mt = (a.M + rows - 1) / rows;
         return dim3((unsigned)((a.nt + 7) / 8 * 8 * a.mt));
     };
     int cols16 = 0;  // 16-column tiles
@@ -590,13 +597,14 @@ void launch_t(Args& a, int M, hipStream_t s) {
 
 size_t gemm_f16_ws_bytes(int K, int M, bool codes) { return planes_of(K, M, !codes).bytes; }
 
-hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t* qa, int K, int M, void* ws,
-                                hipStream_t s) {
-    const Planes pl = planes_of(K, M, mode == 0);
+hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t* qa, const float* bs, int K, int M,
+                                void* ws, hipStream_t s) {
+    const Planes pl = planes_of(K, M, mode == 0 || mode == 3);
     char* b = (char*)ws;
     PrepArgs a{};
     a.A = A;
     a.QA = qa;
+    a.bs = bs;
     a.lda = lda;
     a.M = M;
     a.K = K;
@@ -608,12 +616,13 @@ hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t*
     a.rs = (float*)(b + pl.rs);
     if (mode == 0) launch_prep<0>(a, s);
     else if (mode == 1) launch_prep<1>(a, s);
-    else launch_prep<2>(a, s);
+    else if (mode == 2) launch_prep<2>(a, s);
+    else launch_prep<3>(a, s);
     return hipGetLastError();
 }
 
-hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, bool codes, const float* sa,
-                           const void* ws, hipStream_t s) {
+hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, int M_call, bool codes,
+                           const float* sa, const void* ws, hipStream_t s) {
     if (n < 1 || n > kProb) return hipErrorInvalidValue;
     const Planes pl = planes_of(K, M, !codes);
     const char* b = (const char*)ws;
@@ -627,10 +636,10 @@ hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M
     a.XL = (const h8*)(b + pl.xl);
     a.XS = (const h8*)(b + pl.xs);
     a.rs = sa ? sa : (const float*)(b + pl.rs);
-#define GO(TT)                                   \
-    case TT:                                     \
-        if (codes) launch_t<TT, 1>(a, M, s);     \
-        else launch_t<TT, 2>(a, M, s);           \
+#define GO(TT)                                    \
+    case TT:                                      \
+        if (codes) launch_t<TT, 1>(a, M_call, s); \
+        else launch_t<TT, 2>(a, M_call, s);       \
         break
     switch (type) {
         GO(T_Q4_K);

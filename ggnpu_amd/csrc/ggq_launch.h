@@ -151,13 +151,16 @@ hipError_t launch_gemm_panel(uint32_t type, const GemmDesc* d, int n, int K, con
 // (gemm_f16_ws_bytes, 256-byte aligned; codes: one plane, else two): mode 0
 // fp32 rows A [M][lda], 1 the same quantized per row (codes and scales of
 // launch_quant_act mode 1), 2 given int8 codes qa [M][K] (8-byte aligned,
-// row scales `sa` passed to launch_gemm_f16).  launch_gemm_f16 multiplies
-// them with up to 4 weights of one type.
+// row scales `sa` passed to launch_gemm_f16), 3 given int8 codes and a scale
+// bs [M][K / 32] per 32 values, as the fp32 rows of their products.
+// launch_gemm_f16 multiplies them with up to 4 weights of one type; `M_call`:
+// the rows of the whole call, which choose kernel and tile, so that a result
+// does not depend on the passes that its rows are taken in.
 size_t gemm_f16_ws_bytes(int K, int M, bool codes);
-hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t* qa, int K, int M, void* ws,
-                                hipStream_t s);
-hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, bool codes, const float* sa,
-                           const void* ws, hipStream_t s);
+hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t* qa, const float* bs, int K, int M,
+                                void* ws, hipStream_t s);
+hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, int M_call, bool codes,
+                           const float* sa, const void* ws, hipStream_t s);
 // The same products for few fp32 rows (1..32, A 16-byte aligned, lda % 4 ==
 // 0), which are split in registers, not in planes (ggq_gemm_rows.hip): up to 8
 // weights of any types in one launch.  `ws`: gemm_rows_ws_bytes(K, M, columns

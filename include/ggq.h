@@ -166,8 +166,8 @@ int ggq_mul_mat_dev(ggq_ctx* ctx, const void* W, uint32_t type, int64_t N, int64
  * before queuing anything, while work an earlier eager call queued on
  * another stream is unfinished (calls queued under graph capture are not
  * tracked).  The region's address is looked up on the first call on a
- * device; if that fails only this entry point fails.  Results equal
- * ggq_mul_mat_dev's. */
+ * device; if that fails only this entry point fails.  Results equal those of
+ * ggq_mul_mat_dev with its buffers at hand, bit for bit. */
 #define GGQ_NOALLOC_SCRATCH_BYTES (32u << 20)
 int ggq_mul_mat_noalloc_dev(ggq_ctx* ctx, const void* W, uint32_t type, int64_t N, int64_t K,
                             const float* A, int lda, float* C, int ldc, int M, int act_mode, void* stream);

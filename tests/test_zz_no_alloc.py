@@ -64,6 +64,34 @@ def test_noalloc_matches_mul_mat_dev(ctx, orc, t, N, K, M1, M2, mode):
             assert orc.rel_l2(got, orc.mul_mat_f64(t, raw, N, K, A, mode)) < 1e-4
 
 
+# (type, N, K, M, act mode) whose scratch beside the inputs is more than the region: the rows' planes in passes of
+# rows, the slices' sums of few rows in turns of columns
+MANY = [(12, 96, 8192, 1023, 0), (14, 80, 16384, 600, 0), (8, 96, 8192, 1023, 0), (14, 96, 8192, 2100, 1),
+        (13, 160, 16384, 380, 2), (23, 1040, 8192, 150, 2), (12, 131120, 2304, 32, 0)]
+
+
+@pytest.mark.parametrize("t,N,K,M,mode", MANY)
+def test_noalloc_matches_mul_mat_dev_in_passes(ctx, orc, t, N, K, M, mode):
+    import torch
+    rng = np.random.default_rng(N + K + M)
+    raw = gl.encode(t, (rng.standard_normal((min(N, 523), K)) * 0.02).astype(np.float32))
+    raw = np.resize(raw, N * gl.row_bytes(t, K))  # rows repeat where there are many
+    dW = dev(raw)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    x = torch.zeros((M, K + 4), device="cuda")
+    x[:, :K].copy_(torch.from_numpy(A))
+    y = [torch.full((M, N + 3), 7.0, device="cuda") for _ in range(2)]
+    for out, fn in zip(y, (ctx.lib.ggq_mul_mat_noalloc_dev, ctx.lib.ggq_mul_mat_dev)):
+        ctx.check(fn(ctx.h, ctypes.c_void_p(dW.data_ptr()), t, N, K, ctypes.c_void_p(x.data_ptr()), K + 4,
+                     ctypes.c_void_p(out.data_ptr()), N + 3, M, mode, stream_handle()), fn.__name__)
+    got, exp = host(y[0]), host(y[1])
+    assert np.array_equal(got.view(np.uint32), exp.view(np.uint32)) and (got[:, N:] == 7.0).all()
+    rows = np.unique(np.r_[0, M - 1, np.arange(127, M, 128), np.arange(128, M, 128)])  # both sides of every pass
+    cols = np.unique(np.r_[0:16, N - 16:N])
+    ref = orc.mul_mat_f64(t, raw.reshape(N, -1)[cols].reshape(-1), len(cols), K, A[rows], mode)
+    assert orc.rel_l2(got[rows][:, cols], ref) < 4e-7 + 2.0 ** -24 * np.sqrt(3 * K / 16)  # as in test_gpu_gemm_f16
+
+
 def test_noalloc_rejects_oversized_scratch(ctx):
     import torch
     t, N, K, M = 8, 256, 8192, 4608  # 37.7 MB of int8 activations > the 32 MiB region
