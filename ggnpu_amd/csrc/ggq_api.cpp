@@ -488,8 +488,8 @@ size_t q8_rows_bytes(int K, int M) { return align256((size_t)M * K) + align256(s
 // The workspace that int8 rows need without planes.  Eager calls keep it sized
 // though they do not use it, so that a capture after them that finds no planes
 // left records the int8 GEMMs and is not refused.  (A fixed region has to hold
-// it, though the call does without: what its entry point refuses does not
-// depend on the kernel.)
+// it where it does not hold the planes of all rows: passes over them do not
+// widen what its entry point accepts.)
 int size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M) {
     size_t ws_bytes = 0, part_bytes = 0;
     int Ns[GGQ_MAX_BATCH];
@@ -515,7 +515,9 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
               int lda, const int8_t* qa, const float* sa, int M, hipStream_t s, int* st) {
     const bool codes = mode == GEMM_Q8_ROW || mode == GEMM_CODES;
     const int step = gemm_rows_per_pass(K, M, codes, ar.room(ws_bytes));
-    if (codes && ar.w != &c->host && (*st = size_int8_gemm(c, ar, d, n, K, mode, A, lda, M)) != GGQ_OK && !ar.w) return true;
+    if (codes && (ar.w == &c->dev || step < M) && ar.w != &c->host &&
+        (*st = size_int8_gemm(c, ar, d, n, K, mode, A, lda, M)) != GGQ_OK && !ar.w)
+        return true;
     void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
     if (!ws) return false;
     hipError_t e = hipSuccess;

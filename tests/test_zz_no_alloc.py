@@ -107,6 +107,19 @@ def test_noalloc_rejects_oversized_scratch(ctx):
     assert bool((y == 7.0).all())  # nothing was queued
 
 
+@pytest.mark.parametrize("t", [12, 14])
+def test_noalloc_rejects_oversized_scratch_of_many_rows(ctx, t):
+    """Also where the rows' planes could go in passes: the int8 GEMM's codes exceed the region."""
+    import torch
+    N, K, M = 64, 8192, 4608
+    dW = dev(gl.encode(t, np.zeros((N, K), np.float32)))
+    x, y = torch.zeros((M, K), device="cuda"), torch.full((M, N), 7.0, device="cuda")
+    st = ctx.lib.ggq_mul_mat_noalloc_dev(ctx.h, ctypes.c_void_p(dW.data_ptr()), t, N, K, ctypes.c_void_p(x.data_ptr()),
+                                         K, ctypes.c_void_p(y.data_ptr()), N, M, 1, stream_handle())
+    torch.cuda.synchronize()
+    assert st == int(gl.Status.INVALID_PARAM) and bool((y == 7.0).all())
+
+
 def test_noalloc_refuses_overlap_on_another_stream(ctx):
     """A call whose region is still in use by an unfinished call on another
     stream is refused (nothing queued); once that work is done, or on the
