@@ -357,23 +357,47 @@ template <int PB, int NP> struct Col<T_IQ4_XS, PB, NP> {
     }
 };
 
-// End of a superblock for one tile: its chain P under the column's scale and
-// the mins onto the sums (sm: the sums of x).
-template <int AP, class C, class V>
-__device__ __forceinline__ void close(const C& col, h8 mn, h8 mid, h8 sm, V P, V& acc) {
-    constexpr int E = sizeof(V) / 4;
+template <int CTRL> __device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+// 2^(b - 127), b byte e of the words; 1 in kRowPower.
+constexpr uint32_t kRowPower = 0x7F7F7F7Fu;
+template <int W> __device__ __forceinline__ float power(const uint32_t (&w)[W], int e) {
+    const uint32_t v = w[e >> 2];
+    return __builtin_bit_cast(float, ((e & 3) == 3 ? v >> 1 : v << (23 - 8 * (e & 3))) & 0x7F800000u);
+}
+// End of a superblock for one tile.  with_mins: the chain P of fp32 rows under
+// the column's scale with the mins (sm: the sums of x); they cancel in part, so
+// they meet before they round against the sum.
+template <class C, class V>
+__device__ __forceinline__ void with_mins(const C& col, h8 mn, h8 mid, h8 sm, V& P) {
     const float d = col.k.d, dm = -32.0f * col.k.dm;  // the sums carry 1 / 32
-    if constexpr (C::kMin) {
-        if constexpr (AP == 2) P = mfma(sm, mid, P);
-        const V S = mfma(sm, mn, V{});
-        // codes: both are exact integers; rows: P and S cancel in part, so they
-        // meet before they round against the sum
+    P = mfma(sm, mid, P);
+    const V S = mfma(sm, mn, V{});
 #pragma unroll
-        for (int e = 0; e < E; e++)
-            acc[e] = AP == 2 ? acc[e] + __builtin_fmaf(d, P[e], dm * S[e]) : __builtin_fmaf(d, P[e], __builtin_fmaf(dm, S[e], acc[e]));
+    for (int e = 0; e < (int)sizeof(V) / 4; e++) P[e] = __builtin_fmaf(d, P[e], dm * S[e]);
+}
+// close: the same and the chains without mins onto the sums; times(e, v): v
+// under the power of two of element e's row.
+struct NoPower {
+    __device__ __forceinline__ float operator()(int, float v) const { return v; }
+};
+template <int AP, class C, class V, class F = NoPower>
+__device__ __forceinline__ void close(const C& col, h8 mn, h8 mid, h8 sm, V P, V& acc, F times = NoPower{}) {
+    constexpr int E = sizeof(V) / 4;
+    const float d = col.k.d;
+    if constexpr (C::kMin && AP == 2) {
+        with_mins(col, mn, mid, sm, P);
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[e] += times(e, P[e]);
+    } else if constexpr (C::kMin) {  // codes: both are exact integers
+        const float dm = -32.0f * col.k.dm;
+        const V S = mfma(sm, mn, V{});
+#pragma unroll
+        for (int e = 0; e < E; e++) acc[e] = __builtin_fmaf(d, P[e], __builtin_fmaf(dm, S[e], acc[e]));
     } else {
 #pragma unroll
-        for (int e = 0; e < E; e++) acc[e] = __builtin_fmaf(d, P[e], acc[e]);
+        for (int e = 0; e < E; e++) acc[e] = __builtin_fmaf(d, times(e, P[e]), acc[e]);
     }
 }
 template <int AP, class C>

@@ -3,9 +3,13 @@
 // cores of gfx950; the weights as ggq_cols.h decodes them.
 //
 // Activations.  prep_* kernels write them once as fp16 planes in the order
-// the MFMA reads: fp32 rows as hi + lo under a power of two per row (22
-// bits), int8 codes as one exact plane.  For codes every product and, below
-// 2^24, every partial sum of a superblock is an exact integer in fp32.
+// the MFMA reads: fp32 rows as hi + lo (22 bits) under a power of two per row
+// and superblock, int8 codes as one exact plane.  A power per row alone lost the
+// values that lie far below a row's largest (rows with one value of 2^22 in a
+// superblock of zero weights, K = 8192, 48 rows, Q5_K: relative error 8.3e-6;
+// with a power per superblock 2.1e-7, fp32 FMA 2.3e-7).  For codes every product
+// and, below 2^24, every partial sum of a superblock is an exact integer in
+// fp32.
 // The planes are stored in the piece order of the 32x32x16 MFMA, [32-row
 // tile][step 2g + u][lane][8]; the 16x16x32 one's operand is four runs of 256
 // bytes of it.
@@ -15,6 +19,7 @@ namespace ggq {
 namespace {
 
 constexpr int kProb = 4;
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 struct Prob {
     const uint8_t* W;
     float* C;
@@ -28,7 +33,8 @@ struct Args {
     const h8* XH;
     const h8* XL;
     const h8* XS;
-    const float* rs;  // scale of each row
+    const uint32_t* XE;  // powers of two of each row and superblock (fp32 rows)
+    const float* rs;     // scale of each row
 };
 
 __device__ __forceinline__ void store(const Args& a, const Prob& p, int m, int n, float v) {
@@ -88,6 +94,11 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f16_ks_kernel(Args a) {
         const h8 v = a.XS[((size_t)(r >> 1) * a.SB + sb) * 64 + 32 * (q & 1) + 16 * (r & 1) + (lane & 15)];
         return q < 2 ? v : h8{};
     };
+    // powers of the lane's four rows
+    auto powers = [&](int i, int sb, uint32_t (&e)[1]) {
+        const int r = m0 / 16 + i;
+        e[0] = a.XE[((size_t)(r >> 1) * a.SB + sb) * 8 + 4 * (q & 1) + 2 * (r & 1) + (q >> 1)];
+    };
 
     f4v acc[MF][NF];
 #pragma unroll
@@ -119,13 +130,17 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f16_ks_kernel(Args a) {
         const int nsb = sb + KW < a.SB ? sb + KW : sb;
         f4v P[MF][NF];
         h8 sm[MF];
+        uint32_t pw[MF][1];
 #pragma unroll
         for (int j = 0; j < NF; j++) {
             col[j].open(sb, q, a.nb);
             col[j].load_head(row[j], nsb, q, a.nb);
         }
 #pragma unroll
-        for (int i = 0; i < MF; i++) sm[i] = C::kMin ? sums(i, sb) : h8{};
+        for (int i = 0; i < MF; i++) {
+            sm[i] = C::kMin ? sums(i, sb) : h8{};
+            if constexpr (AP == 2) powers(i, sb, pw[i]);
+        }
 #pragma unroll
         for (int g = 0; g < 8; g++) {
             Frag f[NF];
@@ -161,7 +176,10 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f16_ks_kernel(Args a) {
             h8 mn, mid;
             min_operands<AP>(col[j], mn, mid);
 #pragma unroll
-            for (int i = 0; i < MF; i++) close<AP>(col[j], mn, mid, sm[i], P[i][j], acc[i][j]);
+            for (int i = 0; i < MF; i++) {
+                if constexpr (AP == 2) close<AP>(col[j], mn, mid, sm[i], P[i][j], acc[i][j], [&](int e, float v) { return power(pw[i], e) * v; });
+                else close<AP>(col[j], mn, mid, sm[i], P[i][j], acc[i][j]);
+            }
         }
     }
 
@@ -195,15 +213,28 @@ __device__ __forceinline__ void dma16(const h8* src, uint32_t lane16, uint32_t l
 // Q6_K 394 -> 215 us (registers: that shape spilled).  Operands of a step are
 // read during the step before it; weights straight from the caches, one part
 // ahead.
+constexpr int kRing = 4;  // chunks
+// Workgroups of a CU, by their LDS.
+template <int AP, int MF, int NWN, int CS> constexpr int ring_wgs() {
+    return 4 / NWN * kRing * MF * AP * CS * 1024 <= 64 * 1024 ? 2 : 1;
+}
+// Superblocks of the longest row of a ring kernel; more need more K slices.
+constexpr int kMaxSB = 128;
+template <int NWN> constexpr int ring_sb() { return NWN == 4 ? 16 : NWN == 2 ? 32 : kMaxSB; }
 template <int T, int AP, int MF, int NF, int NWN, int CS>
-__global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
-    constexpr int PB = 2, KW = 4 / NWN, S = 4, R = MF * NF * 16;
+__global__ __launch_bounds__(256, (ring_wgs<AP, MF, NWN, CS>())) void gemm_f16_ring_kernel(Args a) {
+    constexpr int PB = 2, KW = 4 / NWN, S = kRing, R = MF * NF * 16;
     constexpr int CB = MF * AP * CS * 64;  // h8 of a chunk
     constexpr int PP = MF * AP * CS / NWN;  // loads of a wavefront per chunk
     constexpr int NC = 16 / CS;             // chunks of a superblock
     static_assert(NC % S == 0, "a superblock's chunks fill whole rounds of the ring");
     constexpr int kRed = KW > 1 ? 4 * R * 64 * 4 / 16 : 0;
-    __shared__ h8 lds[KW * S * CB > kRed ? KW * S * CB : kRed];
+    constexpr int kLds = KW * S * CB > kRed ? KW * S * CB : kRed;
+    // behind the ring, the rows' powers for the whole K (a load near its use
+    // would wait, in order, for the ring's: 2048 x 8192 Q6_K, 500 rows 81 -> 85
+    // us).  Two workgroups stay below 160 KB: at 160 they took turns (18 -> 30).
+    __shared__ h8 lds[kLds + (AP == 2 ? MF * ring_sb<NWN>() * 2 : 0)];
+    u4v* const powers = (u4v*)(lds + kLds);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int nw = w % NWN, kw = w / NWN;
     int mt, nt, pi;
@@ -242,6 +273,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
 #pragma unroll
         for (int j = 0; j < NF; j++) acc[i][j] = f16v{};
     typedef Col<T, PB, 2> C;
+    const int tid = threadIdx.x, ne = a.SB * 2;  // 16 bytes of a row tile
+    u4v pv[AP == 2 ? MF : 1];
+    if constexpr (AP == 2) {
+        static_assert(ring_sb<NWN>() * 2 <= 256, "a row tile's powers in one load");
+        const u4v* src = (const u4v*)a.XE + (size_t)(m0 / 32) * ne + (tid < ne ? tid : 0);
+#pragma unroll
+        for (int k = 0; k < MF; k++) pv[k] = src[ne * k];
+    }
     C col[NF];
     const uint32_t k1024 = opaque(0x64006400u);
     {
@@ -251,6 +290,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
             col[j].load_head(row[j], sb, 2 * h, a.nb);
 #pragma unroll
             for (int c = 0; c < (T == T_Q6_K ? 4 : PB); c++) col[j].load_part(row[j], sb, 2 * h, a.nb, c);
+        }
+    }
+    if constexpr (AP == 2) {  // (waits for its own loads, the first, and none of the ring's)
+        if (tid < ne) {
+#pragma unroll
+            for (int k = 0; k < MF; k++) powers[tid + ne * k] = pv[k];
         }
     }
 #pragma unroll
@@ -263,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
 #pragma unroll
             for (int p = 0; p < AP; p++) xa[t & 1][i][p] = src[((i * AP + p) * CS + t % CS) * 64];
     };
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * PP) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 1) * PP) : "memory");
     read(0);
     for (int it = 0; it < iters; it++) {
         const int sb0 = kw + KW * it;
@@ -330,12 +375,52 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_ring_kernel(Args a) {
             __builtin_amdgcn_sched_barrier(0x6);
         }
         if (!live) continue;
+        // (K-quants of fp32 rows: products and mins are added first, then
+        // scaled where a row's power differs: most superblocks have it)
+        if constexpr (AP == 2) {
+            if constexpr (C::kMin) {
 #pragma unroll
-        for (int j = 0; j < NF; j++) {
-            h8 mn, mid;
-            min_operands<AP>(col[j], mn, mid);
+                for (int j = 0; j < NF; j++) {
+                    h8 mn, mid;
+                    min_operands<AP>(col[j], mn, mid);
 #pragma unroll
-            for (int i = 0; i < MF; i++) close<AP>(col[j], mn, mid, sm[i], P[i][j], acc[i][j]);
+                    for (int i = 0; i < MF; i++) with_mins(col[j], mn, mid, sm[i], P[i][j]);
+                }
+            }
+            uint32_t pw[MF][4], other = 0;
+#pragma unroll
+            for (int i = 0; i < MF; i++) {
+                const u4v e = powers[(i * a.SB + sb) * 2 + h];
+#pragma unroll
+                for (int k = 0; k < 4; k++) pw[i][k] = e[k];
+            }
+#pragma unroll
+            for (int i = 0; i < MF; i++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) other |= pw[i][k] ^ kRowPower;
+            if (__ballot(other != 0)) {
+#pragma unroll
+                for (int i = 0; i < MF; i++)
+#pragma unroll
+                    for (int j = 0; j < NF; j++)
+#pragma unroll
+                        for (int e = 0; e < 16; e++) P[i][j][e] *= power(pw[i], e);
+            }
+#pragma unroll
+            for (int i = 0; i < MF; i++)
+#pragma unroll
+                for (int j = 0; j < NF; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        acc[i][j][e] = C::kMin ? acc[i][j][e] + P[i][j][e] : __builtin_fmaf(col[j].k.d, P[i][j][e], acc[i][j][e]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NF; j++) {
+                h8 mn, mid;
+                min_operands<AP>(col[j], mn, mid);
+#pragma unroll
+                for (int i = 0; i < MF; i++) close<AP>(col[j], mn, mid, sm[i], P[i][j], acc[i][j]);
+            }
         }
     }
     // the last (repeated) loads land before the ring is reused or the workgroup ends
@@ -381,9 +466,15 @@ struct PrepArgs {
     h8* XH;
     h8* XL;
     _Float16* XS;
+    uint8_t* XE;
     float* rs;
 };
 constexpr int kPi[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+// e of the power 2^e that brings the largest magnitude into [2^14, 2^15)
+__device__ __forceinline__ int scale_exp(float amax) {
+    const int ex = 15 - __builtin_amdgcn_frexp_expf(amax);
+    return ex > 126 ? 126 : ex;
+}
 
 // MODE 0: fp32 rows as hi + lo; 1: fp32 rows quantized per row to int8 codes
 // (the codes and scales of the row quantizer); 2: given int8 codes; 3: given
@@ -393,6 +484,7 @@ constexpr int kPi[8] = {0, 2, 1, 3, 4, 6, 5, 7};
 // side by side in the planes (16 RW bytes a run; with a row per workgroup each
 // lane's 16 bytes go to another line).  RP pieces a thread stay in registers
 // between the row's maximum and the conversion; longer rows are read twice.
+// A superblock's pieces lie in one wavefront, PP neighbours in a lane.
 template <int MODE, int RW, int RP, bool VEC>
 __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
     constexpr bool kCodes = MODE >= 2, kSplit = MODE == 0 || MODE == 3;
@@ -405,11 +497,14 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
     const int64_t row = (int64_t)(m < a.M ? m : a.M - 1) * (kCodes ? a.K : a.lda);
     const size_t tile = (size_t)(m >> 5) * a.SB;
     const int r = m & 31, chunk = ps * RP;
+    constexpr int PP = RW == 1 ? 1 : 2;
+    static_assert(RP % PP == 0, "");
+    auto piece = [&](int i) { return PP * (p0 + ps * (i / PP)) + i % PP; };  // of a chunk, register i
     float v[RP][8];
     auto load = [&](int c) {
 #pragma unroll
         for (int i = 0; i < RP; i++) {
-            const int k = 8 * (c + p0 + ps * i);
+            const int k = 8 * (c + piece(i));
             const bool in = m < a.M && k < a.K;
             // no branch around the loads: places past the row read its start
             const int64_t at = row + (in ? k : 0);
@@ -452,11 +547,7 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
         __syncthreads();
         for (int o = 0; o < waves; o++) amax = fmaxf(amax, wmax[o * RW + tid % RW]);
         if constexpr (kSplit) {
-            if (amax > 0.0f) {  // the largest magnitude into [2^14, 2^15)
-                int x2;
-                (void)frexpf(amax, &x2);
-                ex = 15 - x2 > 126 ? 126 : 15 - x2;
-            }
+            if (amax > 0.0f) ex = scale_exp(amax);
             if (tid < RW && m < a.M) a.rs[m] = ldexpf(1.0f, -ex);
         } else {
             const float sc = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
@@ -467,28 +558,55 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
     }
     for (int c = 0;;) {
 #pragma unroll
-        for (int i = 0; i < RP; i++) {
-            const int p = c + p0 + ps * i;
-            if (p >= np) break;
-            h8 hi, lo;
+        for (int i0 = 0; i0 < RP; i0 += PP) {
+            const int q0 = c + piece(i0), g = q0 >> 2, h = (q0 >> 1) & 1;
+            if (q0 >= np) break;
+            int es = ex;
+            if constexpr (kSplit) {
+                float smax = 0.0f;
+#pragma unroll
+                for (int j = 0; j < PP; j++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) smax = fmaxf(smax, fabsf(v[i0 + j][e]));
+                // the other pieces: in the sixteen lanes, then in the others
+                if constexpr (RW == 1) {
+                    smax = fmaxf(smax, dpp<0x121>(smax));
+                    smax = fmaxf(smax, dpp<0x122>(smax));
+                }
+                smax = fmaxf(smax, dpp<0x124>(smax));
+                smax = fmaxf(smax, dpp<0x128>(smax));
+                smax = fmaxf(smax, __shfl_xor(smax, 16, 64));
+                if constexpr (RW == 4) smax = fmaxf(smax, __shfl_xor(smax, 32, 64));
+                // its own from 2^4 below the row's on, at most 2^126 from it (a
+                // byte, an fp32 exponent)
+                if (smax > 0.0f && scale_exp(smax) - ex >= 4) es = min(scale_exp(smax), ex + 126);
+                if ((q0 & 31) == 0) a.XE[(tile + (g >> 3)) * 32 + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)] = (uint8_t)(127 - (es - ex));
+            }
             float gs = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float x = v[i][kPi[e]];
-                const float y = kSplit ? ldexpf(x, ex) : MODE == 1 ? (float)to_i8(__fmul_rn(x, inv)) : x;
-                hi[e] = (_Float16)y;
-                lo[e] = (_Float16)(y - (float)hi[e]);
-                gs += kSplit ? (float)hi[e] + (float)lo[e] : y;
+            for (int j = 0; j < PP; j++) {
+                h8 hi, lo;
+                float ps8 = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float x = v[i0 + j][kPi[e]];
+                    const float y = kSplit ? ldexpf(x, es) : MODE == 1 ? (float)to_i8(__fmul_rn(x, inv)) : x;
+                    hi[e] = (_Float16)y;
+                    lo[e] = (_Float16)(y - (float)hi[e]);
+                    ps8 += kSplit ? (float)hi[e] + (float)lo[e] : y;
+                }
+                const int u = (q0 + j) & 1;
+                const size_t at = (tile * 16 + 2 * g + u) * 64 + 32 * h + r;
+                a.XH[at] = hi;
+                if constexpr (kSplit) a.XL[at] = lo;
+                gs += ps8;
             }
-            const int g = p >> 2, h = (p >> 1) & 1, u = p & 1;
-            const size_t at = (tile * 16 + 2 * g + u) * 64 + 32 * h + r;
-            a.XH[at] = hi;
-            if constexpr (kSplit) a.XL[at] = lo;
-            gs += __shfl_xor(gs, RW, 64);  // the group's four pieces: all of them are in this loop
-            gs += __shfl_xor(gs, 2 * RW, 64);
+            // the group's four pieces: all of them are in this loop
+            if constexpr (PP == 1) gs += __shfl_xor(gs, RW, 64);
+            gs += __shfl_xor(gs, 2 * RW / PP, 64);
             const float y = gs * 0.03125f;
             const _Float16 sh = (_Float16)y, sl = (_Float16)(y - (float)sh);
-            if (u == 0) a.XS[((tile + (g >> 3)) * 64 + 32 * h + r) * 8 + (g & 7)] = h ? sl : sh;
+            if ((q0 & 1) == 0) a.XS[((tile + (g >> 3)) * 64 + 32 * h + r) * 8 + (g & 7)] = h ? sl : sh;
         }
         c += chunk;
         if (c >= np) break;
@@ -519,7 +637,7 @@ void launch_prep(const PrepArgs& a, hipStream_t s) {
 
 // Planes of one set of activation rows in a workspace.
 struct Planes {
-    size_t xh, xl, xs, rs, bytes;
+    size_t xh, xl, xs, xe, rs, bytes;
 };
 Planes planes_of(int K, int M, bool two) {
     const size_t rows = ((size_t)M + 127) & ~size_t(127), sb = ((size_t)K + 255) / 256;
@@ -527,7 +645,8 @@ Planes planes_of(int K, int M, bool two) {
     p.xh = 0;
     p.xl = p.xh + rows * sb * 512;
     p.xs = p.xl + (two ? rows * sb * 512 : 0);
-    p.rs = p.xs + rows * sb * 32;
+    p.xe = p.xs + rows * sb * 32;
+    p.rs = p.xe + (two ? rows * sb : 0);
     p.bytes = p.rs + rows * 4;
     return p;
 }
@@ -573,10 +692,10 @@ void launch_t(Args& a, int M, hipStream_t s) {  // M: the rows of the whole call
         else if (rows == 32) KS(2, 8);
         else KS(4, 8 / AP);
 #undef KS
-    } else if ((Col<T, 2, 2>::kTwo || M > 64) && m128 * cols32 >= 8 * kCus && a.SB <= 16) {
+    } else if ((Col<T, 2, 2>::kTwo || M > 64) && m128 * cols32 >= 8 * kCus && a.SB <= ring_sb<4>()) {
         const dim3 g = tiles(128, 128);
         gemm_f16_ring_kernel<T, AP, 4, 1, 4, 4 / AP><<<g, 256, 0, s>>>(a);
-    } else if (m128 * cols32 >= 2 * kCus && a.SB <= 32) {
+    } else if (m128 * cols32 >= 2 * kCus && a.SB <= ring_sb<2>()) {
         if constexpr (Col<T, 2, 2>::kTwo) {
             const dim3 g = tiles(64, 128);
             gemm_f16_ring_kernel<T, AP, 4, 1, 2, 2 / AP><<<g, 256, 0, s>>>(a);
@@ -613,6 +732,7 @@ hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t*
     a.XH = (h8*)(b + pl.xh);
     a.XL = (h8*)(b + pl.xl);
     a.XS = (_Float16*)(b + pl.xs);
+    a.XE = (uint8_t*)(b + pl.xe);
     a.rs = (float*)(b + pl.rs);
     if (mode == 0) launch_prep<0>(a, s);
     else if (mode == 1) launch_prep<1>(a, s);
@@ -623,7 +743,7 @@ hipError_t launch_gemm_f16_prep(int mode, const float* A, int lda, const int8_t*
 
 hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M, int M_call, bool codes,
                            const float* sa, const void* ws, hipStream_t s) {
-    if (n < 1 || n > kProb) return hipErrorInvalidValue;
+    if (n < 1 || n > kProb || K > 256 * kMaxSB) return hipErrorInvalidValue;
     const Planes pl = planes_of(K, M, !codes);
     const char* b = (const char*)ws;
     Args a{};
@@ -635,6 +755,7 @@ hipError_t launch_gemm_f16(uint32_t type, const GemmDesc* d, int n, int K, int M
     a.XH = (const h8*)(b + pl.xh);
     a.XL = (const h8*)(b + pl.xl);
     a.XS = (const h8*)(b + pl.xs);
+    a.XE = (const uint32_t*)(b + pl.xe);
     a.rs = sa ? sa : (const float*)(b + pl.rs);
 #define GO(TT)                                    \
     case TT:                                      \

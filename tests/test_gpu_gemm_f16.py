@@ -90,6 +90,23 @@ def test_tiles_vs_oracle(ctx, orc, t, act):
         run(ctx, orc, t, *s, act, i)
 
 
+@pytest.mark.parametrize("act", [0, 2])
+@pytest.mark.parametrize("t", TYPES)
+def test_values_far_below_the_rows_largest(ctx, orc, t, act):
+    """Rows whose first superblock is up to 2^60 above the others, against weights
+    that are zero there: the others keep their bits (the tolerance is relative
+    to their share alone)."""
+    import torch
+    for i, (N, K, M) in enumerate([(1000, 4352, 64), (600, 8448, 65), (2060, 1280, 300), (4100, 768, 600), (16500, 512, 520)]):
+        w = np.random.default_rng(i).standard_normal((N, K)).astype(np.float32) * np.float32(0.02)
+        w[:, :256] = 0
+        raw, a = gl.encode(t, w), rows(M, K, 70 + i)
+        a[5:, :256] *= np.exp2(np.arange(M - 5) % 61).astype(np.float32)[:, None]
+        y, dW, x = torch.full((M, N), float("nan"), device="cuda"), dev(raw), torch.from_numpy(a).cuda()
+        ctx.check(ctx.lib.ggq_mul_mat_dev(ctx.h, ptr(dW), t, N, K, ptr(x), K, ptr(y), N, M, act, stream_handle()), "mul_mat")
+        check(orc, host(y), t, raw, N, K, a, act)
+
+
 @pytest.mark.parametrize("t", [12, 13, 14, 23])
 def test_codes_small_vs_oracle(ctx, orc, t):
     for i, s in enumerate(SMALL):
