@@ -107,7 +107,8 @@ struct ggq_ctx {
     Buffer pin;   // pinned host staging of A and C for the synchronous host-pointer entry points
     uint32_t* done = nullptr;  // pinned completion word of the synchronous entry points
     uint32_t done_seq = 0;
-    std::vector<void*> retired;  // outgrown device buffers, freed by ggq_destroy
+    std::vector<void*> retired;  // outgrown device buffers, and the memory of the
+                                 // lanes and of captures, freed by ggq_destroy
     ggq_moe_trace trace{};       // intermediates of the last MoE call
     bool trace_rows = false;     // MoE calls keep their fp32 SwiGLU rows
 };
@@ -175,20 +176,17 @@ void* alloc_beside_captures(size_t bytes) {
     return nullptr;
 }
 
-// At least `bytes` set aside for captures, where the bound allows; `copies` of
-// them when that takes new memory.
-void set_aside(ggq_ctx* c, size_t bytes, size_t copies) {
-    if (c->aside.size - c->aside_used >= bytes || !bytes) return;
+// Bytes to allocate so that at least `bytes` are set aside for captures, with
+// room for `copies` of them; 0 when they are, or when the bound does not allow it.
+size_t aside_short(const ggq_ctx* c, size_t bytes, size_t copies) {
+    if (c->aside.size - c->aside_used >= bytes || !bytes) return 0;
     bytes = align256(bytes);
-    copies = std::min(copies, (kCaptureBytes - c->aside_total) / bytes);
-    if (!copies) return;
-    const size_t sz = copies * bytes;
-    void* p = alloc_beside_captures(sz);
-    if (!p) return;
-    if (c->aside.ptr) c->retired.push_back(c->aside.ptr);
-    c->aside = Buffer{p, sz};
+    return bytes * std::min(copies, (kCaptureBytes - c->aside_total) / bytes);
+}
+void set_aside(ggq_ctx* c, void* p, size_t bytes) {
+    c->aside = Buffer{p, bytes};
     c->aside_used = 0;
-    c->aside_total += sz;
+    c->aside_total += bytes;
 }
 
 void* capture_lane(ggq_ctx* c, hipStream_t s, unsigned long long id, size_t bytes) {
@@ -204,14 +202,22 @@ void* capture_lane(ggq_ctx* c, hipStream_t s, unsigned long long id, size_t byte
     return b.ptr;
 }
 
-// `b` of at least `bytes`; the outgrown allocation stays for work queued on it.
+// `b` of at least `bytes` and what captures of such calls may need, in one
+// allocation (a context's first call pays for it); ggq_destroy frees both, so
+// that work queued on outgrown memory keeps it.
 bool grow_lane(ggq_ctx* c, Buffer& b, size_t bytes) {
-    if (b.size >= bytes) return true;
-    const size_t sz = std::max(bytes, 2 * b.size);
-    void* p = alloc_beside_captures(sz);
-    if (!p) return false;
-    if (b.ptr) c->retired.push_back(b.ptr);
-    b = Buffer{p, sz};
+    c->lane_need = std::max(c->lane_need, bytes);
+    // for eight captures in a row, two where that would be more than 256 MB
+    const size_t aside = aside_short(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
+    const size_t lane = b.size >= bytes ? 0 : align256(std::max(bytes, 2 * b.size));
+    if (!lane && !aside) return true;
+    char* p = (char*)alloc_beside_captures(lane + aside);
+    const bool both = p;
+    if (!p && lane && aside) p = (char*)alloc_beside_captures(lane);
+    if (!p) return !lane;
+    c->retired.push_back(p);
+    if (lane) b = Buffer{p, lane};
+    if (aside && both) set_aside(c, p + lane, aside);
     return true;
 }
 
@@ -254,9 +260,6 @@ void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
     }
     if (cs != hipStreamCaptureStatusNone)
         return cs == hipStreamCaptureStatusActive && s != hipStreamPerThread ? capture_lane(c, s, id, bytes) : nullptr;
-    // for eight captures in a row, two where that would be more than 256 MB
-    c->lane_need = std::max(c->lane_need, bytes);
-    set_aside(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
     if (s == hipStreamPerThread) return shared_lane(c, s, bytes);
     Lane* l = nullptr;
     for (Lane& x : c->lanes)
@@ -871,13 +874,8 @@ void ggq_destroy(ggq_ctx* c) {
     for (Buffer* b : {&c->dev.ws, &c->dev.part, &c->host.ws, &c->host.part})
         if (b->ptr) hipFree(b->ptr);
     for (void* p : c->retired) hipFree(p);
-    for (Lane& l : c->lanes)
-        if (l.b.ptr) hipFree(l.b.ptr);
-    for (SharedLane& l : c->shared) {
+    for (SharedLane& l : c->shared)
         if (l.ev) hipEventDestroy(l.ev);
-        if (l.b.ptr) hipFree(l.b.ptr);
-    }
-    if (c->aside.ptr) hipFree(c->aside.ptr);
     if (c->io.ptr) hipFree(c->io.ptr);
     if (c->logits.ptr) hipFree(c->logits.ptr);
     if (c->attn.ptr) hipFree(c->attn.ptr);
@@ -1018,7 +1016,11 @@ int ggq_reserve(ggq_ctx* c, int64_t bytes) {
     int st;
     for (Buffer* buf : {&c->dev.ws, &c->dev.part, &c->logits, &c->attn})
         if ((st = grow(c, *buf, b, c->stream, "reserve")) != GGQ_OK) return st;
-    set_aside(c, b, 1);
+    if (const size_t n = aside_short(c, b, 1))
+        if (void* p = alloc_beside_captures(n)) {
+            c->retired.push_back(p);
+            set_aside(c, p, n);
+        }
     return set_status(c, GGQ_OK);
     GGQ_END(c)
 }
