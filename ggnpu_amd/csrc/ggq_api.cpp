@@ -380,11 +380,10 @@ bool gemm_f16_takes(uint32_t type, int64_t cols, int K, int M, int mode) {
     const bool blocks32 = type == GGQ_TYPE_Q8_0 || type == GGQ_TYPE_IQ4_NL;
     const int64_t w = cols * K, work = w * M;
     if (mode == GEMM_F32) {
-        if (fma_only()) return false;
         // (the wavefronts of few columns take long K in turn: 333 x 16384 Q4_K,
         // 48 rows 36 -> 71, Q8_0, 64 rows 49 -> 84)
-        if (blocks32) return M >= 48 && cols * M >= 49152 && work >= (int64_t)256 << 20;
-        return cols * M >= 32768 && work >= (w >= 1 << 22 ? (int64_t)80 << 20 : (int64_t)256 << 20);
+        if (blocks32) return M >= 48 && cols * M >= 49152 && work >= (int64_t)256 << 20 && !fma_only();
+        return cols * M >= 32768 && work >= (w >= 1 << 22 ? (int64_t)80 << 20 : (int64_t)256 << 20) && !fma_only();
     }
     if (type == GGQ_TYPE_Q6_K) return true;
     if (blocks32) return false;
@@ -420,8 +419,8 @@ struct GroupShape {
 //   6.0 -> 7.6, 8.1 -> 7.6, 12 -> 9.5, 3072 x 2048 9.7 -> 13.7, 12 -> 14, 20 ->
 //   16, 8208 x 1536 16 -> 13, 18 -> 13, 36 -> 17.
 constexpr int kRowsMin = 5;
-bool gemm_rows_takes(const GroupShape& g, int K, int M) {
-    if (M < kRowsMin || M > 32 || fma_only()) return false;
+bool gemm_rows_wins(const GroupShape& g, int K, int M) {
+    if (M < kRowsMin || M > 32) return false;
     const int64_t w = g.cols * K, mi = 1 << 20;
     const bool mixed = g.n_types() > 1;
     if (g.types & (1u << GGQ_TYPE_Q8_0 | 1u << GGQ_TYPE_IQ4_NL)) {
@@ -435,6 +434,7 @@ bool gemm_rows_takes(const GroupShape& g, int K, int M) {
     if (M > 16 && !mixed && K <= 4096 && one_plane) return w >= 8 * mi;
     return w >= (mixed && M <= 16 ? 2 : 3) * mi;
 }
+bool gemm_rows_takes(const GroupShape& g, int K, int M) { return gemm_rows_wins(g, K, M) && !fma_only(); }
 bool gemm_rows_takes(uint32_t type, int64_t N, int K, int M) {
     GroupShape g;
     g.add(type, N);

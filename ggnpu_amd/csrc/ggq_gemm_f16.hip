@@ -194,8 +194,11 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_f16_ks_kernel(Args a) {
     }
 }
 
-// 64 lanes' 16 bytes at src + 16 lane into LDS at lds + 16 lane (LDS offsets
-// below 64 KB); the caller waits on the vector memory counter.
+// 64 lanes' 16 bytes at src + 16 lane into LDS at lds + 16 lane (offsets below
+// 128 KB, the largest ring, which the tests run); the caller waits on the vector
+// memory counter.  (m0 is reserved: the compiler keeps nothing in it, sets it
+// right before its own uses, and takes it in no clobber list.  Its builtin for
+// this load would wait for all of them before each read of LDS.)
 __device__ __forceinline__ void dma16(const h8* src, uint32_t lane16, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane16), "s"(src) : "memory");
 }
@@ -228,6 +231,7 @@ __global__ __launch_bounds__(256, (ring_wgs<AP, MF, NWN, CS>())) void gemm_f16_r
     constexpr int PP = MF * AP * CS / NWN;  // loads of a wavefront per chunk
     constexpr int NC = 16 / CS;             // chunks of a superblock
     static_assert(NC % S == 0, "a superblock's chunks fill whole rounds of the ring");
+    static_assert(KW * S * CB * 16 <= 128 * 1024, "offsets of dma16");
     constexpr int kRed = KW > 1 ? 4 * R * 64 * 4 / 16 : 0;
     constexpr int kLds = KW * S * CB > kRed ? KW * S * CB : kRed;
     // behind the ring, the rows' powers for the whole K (a load near its use

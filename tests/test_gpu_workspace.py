@@ -290,3 +290,51 @@ def test_every_stream_runs_the_same_kernels(N, K, M):
                 assert torch.equal(out, ref), i
     finally:
         c.close()
+
+
+# (type, K, M, bytes reserved): the activation-panel GEMM (K <= 2048, no workspace), then the int8 GEMM, whose
+# workspace is reserved with less than the planes would take
+@pytest.mark.parametrize("ty,K,M,reserve", [(12, 2048, 100, 0), (13, 1792, 33, 0), (23, 1792, 100, 0),
+                                            (14, 2048, 100, 500_000), (14, 4352, 33, 1 << 20), (12, 4352, 100, 1 << 20),
+                                            (13, 4352, 33, 1 << 20), (23, 4352, 20, 1 << 20)])
+def test_int8_kernels_without_planes(orc, ty, K, M, reserve):
+    """What captures of int8 rows record when no planes are set aside, through
+    each entry point: against the oracle, fp32 rows and codes bit for bit alike."""
+    import torch
+    N = 72
+    c = gl.Context(0)
+    try:
+        raw = t.weights(ty, N, K, seed=K + ty)
+        W = dev(raw)
+        a = np.random.default_rng(K + M).standard_normal((M, K)).astype(np.float32)
+        x, y = torch.from_numpy(a).cuda(), [torch.zeros((M, N), device="cuda") for _ in range(6)]
+        q, sa = torch.zeros((M, K), dtype=torch.int8, device="cuda"), torch.zeros(M, device="cuda")
+        c.check(c.lib.ggq_quantize_act_dev(c.h, ptr(x), K, M, K, 1, ptr(q), ptr(sa), None), "quantize")
+        c.check(c.lib.ggq_reserve(c.h, reserve), "reserve")
+        gd, bd = (gl.GemmDesc * 2)(), (gl.GemvDesc * 2)()
+        for i in range(2):
+            gd[i].W, gd[i].N, gd[i].C, gd[i].ldc = W.data_ptr(), N, y[2 + i].data_ptr(), N
+            bd[i].W, bd[i].type, bd[i].N, bd[i].K = W.data_ptr(), ty, N, K
+            bd[i].A, bd[i].C = x.data_ptr(), y[4 + i].data_ptr()
+        s = torch.cuda.Stream()
+        h = ctypes.c_void_p(s.cuda_stream)
+        status = []
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        capture(g, s, lambda: status.extend([
+            c.lib.ggq_mul_mat_dev(c.h, ptr(W), ty, N, K, ptr(x), K, ptr(y[0]), N, M, 1, h),
+            c.lib.ggq_mul_mat_q8_dev(c.h, ptr(W), ty, N, K, ptr(q), ptr(sa), M, ptr(y[1]), N, h),
+            c.lib.ggq_mul_mat_q8_batch_dev(c.h, gd, 2, ty, K, ptr(q), ptr(sa), M, h),
+            c.lib.ggq_mul_mat_batch_act_dev(c.h, bd, 2, M, 1, h)]))
+        assert status == [0] * 4, c.lib.ggq_last_error_message(c.h)
+        ref = orc.mul_mat_f64(ty, raw, N, K, a, 1)
+        for _ in range(2):
+            for v in y:
+                v.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            for v in y:
+                assert orc.rel_l2(host(v), ref) < t.TOL
+            assert torch.equal(y[0], y[1])
+    finally:
+        c.close()
