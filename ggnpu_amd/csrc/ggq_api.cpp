@@ -418,6 +418,9 @@ struct GroupShape {
 //   8.2 -> 6.1, 12 -> 9, 4096 x 1024, 5 rows 7.1 -> 6.2; with IQ4_NL, 3072 x 1024
 //   6.0 -> 7.6, 8.1 -> 7.6, 12 -> 9.5, 3072 x 2048 9.7 -> 13.7, 12 -> 14, 20 ->
 //   16, 8208 x 1536 16 -> 13, 18 -> 13, 36 -> 17.
+//   Up to 8 rows with Q8_0 or IQ4_NL the int8 GEMVs win from 24 M weights on:
+//   Q4_K + IQ4_NL, 8 rows, 12288 x 2048 22 -> 23, 16384 x 2048 22 -> 27, 32768 x
+//   2048 33 -> 44 (IQ4_XS + Q8_0, 17920 x 1536 23 -> 17).
 constexpr int kRowsMin = 5;
 bool gemm_rows_wins(const GroupShape& g, int K, int M) {
     if (M < kRowsMin || M > 32) return false;

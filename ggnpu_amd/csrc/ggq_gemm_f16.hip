@@ -203,6 +203,15 @@ __device__ __forceinline__ void dma16(const h8* src, uint32_t lane16, uint32_t l
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(lane16), "s"(src) : "memory");
 }
 
+constexpr int kRing = 4;  // chunks
+// Workgroups of a CU, by their LDS.
+template <int AP, int MF, int NWN, int CS> constexpr int ring_wgs() {
+    return 4 / NWN * kRing * MF * AP * CS * 1024 <= 64 * 1024 ? 2 : 1;
+}
+// Superblocks of the longest row of a ring kernel; more need more K slices.
+constexpr int kMaxSB = 128;
+template <int NWN> constexpr int ring_sb() { return NWN == 4 ? 16 : NWN == 2 ? 32 : kMaxSB; }
+
 // Many tiles: a workgroup of four wavefronts takes 64 rows; NWN of them sit
 // side by side (64 columns each) and share the planes, which the memory
 // system writes into a ring of four LDS slots three chunks (of CS steps)
@@ -213,17 +222,10 @@ __device__ __forceinline__ void dma16(const h8* src, uint32_t lane16, uint32_t l
 // of these MFMAs on random values reaches on this card, 1.1 its library's
 // matmul), the decoding VALU with one (99 us).  128 x 32 values a wavefront
 // decode a weight once per 128 rows: against 64 x 64, one plane 106 -> 99 us,
-// Q6_K 394 -> 215 us (registers: that shape spilled).  Operands of a step are
-// read during the step before it; weights straight from the caches, one part
-// ahead.
-constexpr int kRing = 4;  // chunks
-// Workgroups of a CU, by their LDS.
-template <int AP, int MF, int NWN, int CS> constexpr int ring_wgs() {
-    return 4 / NWN * kRing * MF * AP * CS * 1024 <= 64 * 1024 ? 2 : 1;
-}
-// Superblocks of the longest row of a ring kernel; more need more K slices.
-constexpr int kMaxSB = 128;
-template <int NWN> constexpr int ring_sb() { return NWN == 4 ? 16 : NWN == 2 ? 32 : kMaxSB; }
+// Q6_K 394 -> 215 us (64 x 64 spilled most of its sums; here the fp32 rows of
+// Q6_K still spill 26 registers and those of the other formats up to 7).
+// Operands of a step are read during the step before it; weights straight from
+// the caches, one part ahead.
 template <int T, int AP, int MF, int NF, int NWN, int CS>
 __global__ __launch_bounds__(256, (ring_wgs<AP, MF, NWN, CS>())) void gemm_f16_ring_kernel(Args a) {
     constexpr int PB = 2, KW = 4 / NWN, S = kRing, R = MF * NF * 16;
@@ -655,8 +657,8 @@ Planes planes_of(int K, int M, bool two) {
     return p;
 }
 
-// Kernel and tile of a launch, by how many workgroups each would give the 256
-// CUs (times of 2048 x 2048 / 8192 x 2048 Q4_K, fp32 rows, in us):
+// Kernel and tile of a launch, by how many workgroups each would give the CUs
+// (of 256; times of 2048 x 2048 / 8192 x 2048 Q4_K, fp32 rows, in us):
 //   K split over 8 wavefronts, 16 columns a workgroup, as long as every CU
 //   gets at most one (64 rows: 16 / 29), then 32 columns (19 / 20);
 //   128-row tiles from the ring otherwise: 128 columns a workgroup from two
@@ -671,7 +673,7 @@ Planes planes_of(int K, int M, bool two) {
 // row kernels' 2.35e-7).
 template <int T, int AP>
 void launch_t(Args& a, int M, hipStream_t s) {  // M: the rows of the whole call
-    constexpr int kCus = 256;
+    const int cus = cu_count();
     // tiles of `cols` x `rows`; returns the grid
     auto tiles = [&](int cols, int rows) {
         a.nt = 0;
@@ -685,8 +687,8 @@ void launch_t(Args& a, int M, hipStream_t s) {  // M: the rows of the whole call
     int cols16 = 0;  // 16-column tiles
     for (int i = 0; i < a.np; i++) cols16 += (a.p[i].N + 15) / 16;
     const int cols32 = (cols16 + 1) / 2, m64 = (M + 63) / 64, m128 = (M + 127) / 128;
-    const bool narrow = m64 <= 8 && m64 * cols16 <= kCus;
-    if (narrow || M <= 32 || (m64 <= 4 && m64 * cols32 <= kCus)) {
+    const bool narrow = m64 <= 8 && m64 * cols16 <= cus;
+    if (narrow || M <= 32 || (m64 <= 4 && m64 * cols32 <= cus)) {
         const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
         const dim3 g = tiles(narrow ? 16 : 32, rows);
 #define KS(MF, NB)                                                                       \
@@ -696,10 +698,10 @@ void launch_t(Args& a, int M, hipStream_t s) {  // M: the rows of the whole call
         else if (rows == 32) KS(2, 8);
         else KS(4, 8 / AP);
 #undef KS
-    } else if ((Col<T, 2, 2>::kTwo || M > 64) && m128 * cols32 >= 8 * kCus && a.SB <= ring_sb<4>()) {
+    } else if ((Col<T, 2, 2>::kTwo || M > 64) && m128 * cols32 >= 8 * cus && a.SB <= ring_sb<4>()) {
         const dim3 g = tiles(128, 128);
         gemm_f16_ring_kernel<T, AP, 4, 1, 4, 4 / AP><<<g, 256, 0, s>>>(a);
-    } else if (m128 * cols32 >= 2 * kCus && a.SB <= ring_sb<2>()) {
+    } else if (m128 * cols32 >= 2 * cus && a.SB <= ring_sb<2>()) {
         if constexpr (Col<T, 2, 2>::kTwo) {
             const dim3 g = tiles(64, 128);
             gemm_f16_ring_kernel<T, AP, 4, 1, 2, 2 / AP><<<g, 256, 0, s>>>(a);

@@ -271,7 +271,7 @@ bool gemm_rows_eligible(int K, int M, const float* A, int lda) {
 hipError_t launch_gemm_rows(const GemmDesc* d, const uint32_t* types, int n, int K, const float* A, int lda, int M, void* ws,
                             hipStream_t s) {
     if (n < 1 || n > kProb || !gemm_rows_eligible(K, M, A, lda)) return hipErrorInvalidValue;
-    constexpr int kCus = 256;
+    const int cus = cu_count();
     Args a{};
     a.np = n;
     a.M = M;
@@ -291,7 +291,7 @@ hipError_t launch_gemm_rows(const GemmDesc* d, const uint32_t* types, int n, int
     if (cols > INT32_MAX || (a.slices > 1 && !ws)) return hipErrorInvalidValue;
     // one workgroup of eight wavefronts fills a CU's registers; as many as
     // leave every workgroup the same number of tiles
-    const int64_t cap = kCus * (kWaves / a.per) / a.slices > 1 ? kCus * (kWaves / a.per) / a.slices : 1;
+    const int64_t cap = cus * (kWaves / a.per) / a.slices > 1 ? cus * (kWaves / a.per) / a.slices : 1;
     const int64_t rounds = (tiles + cap - 1) / cap;
     int wg = 0, col0 = 0;
     for (int i = 0; i < n; i++) {

@@ -980,16 +980,6 @@ int env_i8(const char* name, int dflt) {
     return e && *e ? atoi(e) : dflt;
 }
 
-int cu_count() {
-    static int v = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
-    return v;
-}
-
 // Formats with four scale slots per MFMA (one row per pass in fp32 mode).
 bool g4_format(uint32_t t) { return t == T_Q6_K || t == T_IQ4_NL || t == T_IQ4_XS; }
 

@@ -7,6 +7,17 @@
 
 namespace ggq {
 
+// CUs of the device that is current on the first call.
+inline int cu_count() {
+    static int v = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return v;
+}
+
 // Standalone bit-exact dequant of n_blocks consecutive blocks.
 hipError_t launch_dequant(uint32_t type, const void* raw, int64_t n_blocks, float* out, hipStream_t s);
 
