@@ -107,8 +107,8 @@ struct ggq_ctx {
     Buffer pin;   // pinned host staging of A and C for the synchronous host-pointer entry points
     uint32_t* done = nullptr;  // pinned completion word of the synchronous entry points
     uint32_t done_seq = 0;
-    std::vector<void*> retired;  // outgrown device buffers, and the memory of the
-                                 // lanes and of captures, freed by ggq_destroy
+    std::vector<void*> owned;  // device allocations behind the buffers above (outgrown
+                               // ones too), freed by ggq_destroy
     ggq_moe_trace trace{};       // intermediates of the last MoE call
     bool trace_rows = false;     // MoE calls keep their fp32 SwiGLU rows
 };
@@ -155,9 +155,8 @@ int grow(ggq_ctx* c, Buffer& b, size_t need, hipStream_t s, const char* what) {
     void* p = nullptr;
     const hipError_t e = hipMalloc(&p, sz);
     if (e != hipSuccess) return hip_status(c, e, what);
-    if (b.ptr) c->retired.push_back(b.ptr);
-    b.ptr = p;
-    b.size = sz;
+    c->owned.push_back(p);
+    b = Buffer{p, sz};
     return GGQ_OK;
 }
 
@@ -202,27 +201,44 @@ void* capture_lane(ggq_ctx* c, hipStream_t s, unsigned long long id, size_t byte
     return b.ptr;
 }
 
-// `b` of at least `bytes` and what captures of such calls may need, in one
-// allocation (a context's first call pays for it); ggq_destroy frees both, so
-// that work queued on outgrown memory keeps it.
-bool grow_lane(ggq_ctx* c, Buffer& b, size_t bytes) {
+// A buffer that has to grow to at least `bytes` some time, for calls outside
+// captures; none where it is large enough.
+struct Want {
+    Buffer* b;
+    size_t bytes;
+    size_t grown() const { return bytes && b->size < bytes ? align256(std::max(bytes, 2 * b->size)) : 0; }
+};
+
+// `b` of at least `bytes`, with what captures of such calls may need and what
+// the context `wants` by the way, in one allocation (a context's first call pays
+// for it).
+bool grow_lane(ggq_ctx* c, Buffer& b, size_t bytes, const Want* wants, int n_wants) {
     c->lane_need = std::max(c->lane_need, bytes);
     // for eight captures in a row, two where that would be more than 256 MB
     const size_t aside = aside_short(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
-    const size_t lane = b.size >= bytes ? 0 : align256(std::max(bytes, 2 * b.size));
-    if (!lane && !aside) return true;
-    char* p = (char*)alloc_beside_captures(lane + aside);
-    const bool both = p;
-    if (!p && lane && aside) p = (char*)alloc_beside_captures(lane);
+    const size_t lane = Want{&b, bytes}.grown();
+    size_t extra = aside;
+    for (int i = 0; i < n_wants; i++) extra += wants[i].grown();
+    if (!lane && !extra) return true;
+    char* p = (char*)alloc_beside_captures(lane + extra);
+    const bool all = p;
+    if (!p && lane && extra) p = (char*)alloc_beside_captures(lane);
     if (!p) return !lane;
-    c->retired.push_back(p);
+    c->owned.push_back(p);
     if (lane) b = Buffer{p, lane};
-    if (aside && both) set_aside(c, p + lane, aside);
+    if (!all) return true;
+    p += lane;
+    for (int i = 0; i < n_wants; i++)
+        if (const size_t n = wants[i].grown()) {
+            *wants[i].b = Buffer{p, n};
+            p += n;
+        }
+    if (aside) set_aside(c, p, aside);
     return true;
 }
 
 // A shared lane for the call being queued on `s`; lane_done ends its use.
-void* shared_lane(ggq_ctx* c, hipStream_t s, size_t bytes) {
+void* shared_lane(ggq_ctx* c, hipStream_t s, size_t bytes, const Want* wants, int n_wants) {
     SharedLane* l = nullptr;
     for (SharedLane& x : c->shared)
         if (x.ev && x.stream == s) l = &x;
@@ -231,7 +247,7 @@ void* shared_lane(ggq_ctx* c, hipStream_t s, size_t bytes) {
     if (l->ev) e = hipStreamWaitEvent(s, l->ev, 0);
     else if ((e = hipEventCreateWithFlags(&l->ev, hipEventDisableTiming)) != hipSuccess) l->ev = nullptr;
     if (e != hipSuccess) (void)hipGetLastError();
-    if (e != hipSuccess || !grow_lane(c, l->b, bytes)) return nullptr;
+    if (e != hipSuccess || !grow_lane(c, l->b, bytes, wants, n_wants)) return nullptr;
     l->stream = s;
     c->leased = l;
     return l->b.ptr;
@@ -251,7 +267,7 @@ void lane_done(ggq_ctx* c, hipStream_t s) {
 // caller then takes a path without this workspace): no memory, or a capture for
 // which not enough was set aside or whose stream cannot be told from others
 // (hipStreamPerThread: one handle for several).
-void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
+void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes, const Want* wants, int n_wants) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (hipStreamGetCaptureInfo(s, &cs, &id) != hipSuccess) {
@@ -260,17 +276,17 @@ void* lane_ws(ggq_ctx* c, hipStream_t s, size_t bytes) {
     }
     if (cs != hipStreamCaptureStatusNone)
         return cs == hipStreamCaptureStatusActive && s != hipStreamPerThread ? capture_lane(c, s, id, bytes) : nullptr;
-    if (s == hipStreamPerThread) return shared_lane(c, s, bytes);
+    if (s == hipStreamPerThread) return shared_lane(c, s, bytes, wants, n_wants);
     Lane* l = nullptr;
     for (Lane& x : c->lanes)
         if (x.stream == s) l = &x;
     if (!l) {
-        if (c->lanes.size() >= kMaxLanes) return shared_lane(c, s, bytes);
+        if (c->lanes.size() >= kMaxLanes) return shared_lane(c, s, bytes, wants, n_wants);
         c->lanes.emplace_back();
         l = &c->lanes.back();
         l->stream = s;
     }
-    return grow_lane(c, l->b, bytes) ? l->b.ptr : nullptr;
+    return grow_lane(c, l->b, bytes, wants, n_wants) ? l->b.ptr : nullptr;
 }
 
 // Where a call's scratch memory comes from: the growable buffers of a Work,
@@ -303,9 +319,11 @@ struct Arena {
     }
     // Planes of the fp16 GEMM beside `ws_bytes` taken with get(), or null
     // when the call should run without them; planes_done once the work that
-    // uses them is queued.
-    void* planes(size_t ws_bytes, size_t bytes) {
-        if (w == &c->dev) return lane_ws(c, s, bytes);
+    // uses them is queued.  `spare_ws`, `spare_part`: what get() should have
+    // ready for a later capture, outside captures.
+    void* planes(size_t ws_bytes, size_t bytes, size_t spare_ws = 0, size_t spare_part = 0) {
+        const Want wants[2] = {{&c->dev.ws, spare_ws}, {&c->dev.part, spare_part}};
+        if (w == &c->dev) return lane_ws(c, s, bytes, wants, 2);
         if (w) return grow(c, w->part, bytes, s, "workspace") == GGQ_OK ? w->part.ptr : nullptr;
         const size_t off = align256(ws_bytes);
         return off + bytes <= cap ? fixed + off : nullptr;
@@ -491,29 +509,21 @@ int gemm_rows_per_pass(int K, int M, bool codes, size_t room) {
 // Workspace of the int8 GEMM for per-row int8 rows: codes and scales.
 size_t q8_rows_bytes(int K, int M) { return align256((size_t)M * K) + align256(sizeof(float) * (size_t)M * (K / 32)); }
 
-// The workspace that int8 rows need without planes.  Eager calls keep it sized
-// though they do not use it, so that a capture after them that finds no planes
-// left records the int8 GEMMs and is not refused.  (A fixed region has to hold
-// it where it does not hold the planes of all rows: passes over them do not
-// widen what its entry point accepts.)
-int size_int8_gemm(ggq_ctx* c, Arena& ar, const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M) {
-    size_t ws_bytes = 0, part_bytes = 0;
+// The workspace that int8 rows need without planes.
+void int8_gemm_bytes(const GemmEntry* d, int n, int K, int mode, const float* A, int lda, int M, size_t* ws_bytes,
+                     size_t* part_bytes) {
     int Ns[GGQ_MAX_BATCH];
     bool one_type = true;
+    *ws_bytes = *part_bytes = 0;
     for (int i = 0; i < n; i++) {
         Ns[i] = d[i].N;
         one_type = one_type && d[i].type == d[0].type;
         if (ggq::gemm_panel_eligible(d[i].type, K, M, A, lda)) continue;
-        part_bytes = std::max(part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[i].type, &Ns[i], 1, K, M)));
-        if (mode == GEMM_Q8_ROW) ws_bytes = q8_rows_bytes(K, M);
+        *part_bytes = std::max(*part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[i].type, &Ns[i], 1, K, M)));
+        if (mode == GEMM_Q8_ROW) *ws_bytes = q8_rows_bytes(K, M);
     }
-    if (part_bytes && one_type && n > 1 && n <= GGQ_MAX_GEMM_BATCH)
-        part_bytes = std::max(part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[0].type, Ns, n, K, M)));
-    void* ws;
-    float* part;
-    const int st = ar.get(ws_bytes, part_bytes, &ws, &part, "workspace");
-    if (st != GGQ_OK) (void)hipGetLastError();
-    return st;
+    if (*part_bytes && one_type && n > 1 && n <= GGQ_MAX_GEMM_BATCH)
+        *part_bytes = std::max(*part_bytes, gemm_part_bytes(ggq::plan_gemm_i8(d[0].type, Ns, n, K, M)));
 }
 
 // True when the call was taken (*st its status); false: not queued.
@@ -521,10 +531,19 @@ bool gemm_f16(ggq_ctx* c, Arena& ar, size_t ws_bytes, const GemmEntry* d, int n,
               int lda, const int8_t* qa, const float* sa, int M, hipStream_t s, int* st) {
     const bool codes = mode == GEMM_Q8_ROW || mode == GEMM_CODES;
     const int step = gemm_rows_per_pass(K, M, codes, ar.room(ws_bytes));
-    if (codes && (ar.w == &c->dev || step < M) && ar.w != &c->host &&
-        (*st = size_int8_gemm(c, ar, d, n, K, mode, A, lda, M)) != GGQ_OK && !ar.w)
-        return true;
-    void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes));
+    // Eager calls keep the workspace of the int8 GEMM sized though they do not
+    // use it, so that a capture after them that finds no planes left records that
+    // GEMM and is not refused.  A fixed region has to hold it where it does not
+    // hold the planes of all rows: passes over them do not widen what its entry
+    // point accepts.
+    size_t spare_ws = 0, spare_part = 0;
+    if (codes) int8_gemm_bytes(d, n, K, mode, A, lda, M, &spare_ws, &spare_part);
+    if (codes && !ar.w && step < M) {
+        void* p;
+        float* part;
+        if ((*st = ar.get(spare_ws, spare_part, &p, &part, "workspace")) != GGQ_OK) return true;
+    }
+    void* ws = ar.planes(ws_bytes, ggq::gemm_f16_ws_bytes(K, step, codes), spare_ws, spare_part);
     if (!ws) return false;
     hipError_t e = hipSuccess;
     for (int m0 = 0; m0 < M && e == hipSuccess; m0 += step) {
@@ -874,14 +893,9 @@ void ggq_destroy(ggq_ctx* c) {
         hipFree(w->dev);
         delete w;
     }
-    for (Buffer* b : {&c->dev.ws, &c->dev.part, &c->host.ws, &c->host.part})
-        if (b->ptr) hipFree(b->ptr);
-    for (void* p : c->retired) hipFree(p);
+    for (void* p : c->owned) hipFree(p);
     for (SharedLane& l : c->shared)
         if (l.ev) hipEventDestroy(l.ev);
-    if (c->io.ptr) hipFree(c->io.ptr);
-    if (c->logits.ptr) hipFree(c->logits.ptr);
-    if (c->attn.ptr) hipFree(c->attn.ptr);
     if (c->pin.ptr) hipHostFree(c->pin.ptr);
     if (c->done) hipHostFree(c->done);
     hipStreamDestroy(c->stream);
@@ -1021,7 +1035,7 @@ int ggq_reserve(ggq_ctx* c, int64_t bytes) {
         if ((st = grow(c, *buf, b, c->stream, "reserve")) != GGQ_OK) return st;
     if (const size_t n = aside_short(c, b, 1))
         if (void* p = alloc_beside_captures(n)) {
-            c->retired.push_back(p);
+            c->owned.push_back(p);
             set_aside(c, p, n);
         }
     return set_status(c, GGQ_OK);
