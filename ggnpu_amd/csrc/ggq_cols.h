@@ -8,7 +8,8 @@
 // values, hi = fp16(q*s) and the exact remainder lo = q*s - hi (a fused
 // multiply-add), in two planes.  The K-quant mins are one more MFMA per
 // superblock: the sums of x over the 32 values of each sub-block against the
-// 6-bit mins.
+// 6-bit mins.  fp32 rows are hi + lo as well; against two weight planes the
+// product of the two low parts (2^-22 of a product) is left out.
 //
 // Pieces: piece q (0..3) of a 32-value group g holds the values k = 32 g + 8 q
 // + {0,2,1,3,4,6,5,7} of one row or column, one lane's operand of an MFMA.

@@ -18,6 +18,9 @@
 // rows' way into registers: about 6 us for 16 rows, 9 for 32) and past it the
 // decoding VALU, 0.39 us per 1000 columns of K = 2048 (3.0 TB/s of Q4_K; 2.5
 // with 32 rows).
+// Error against 64 bits on N(0, 1) rows, in every format, over that of the fp32
+// kernels (products of 24 bits): 0.8 in the middle and at most 1.0 up to K =
+// 4096, 0.9 and 1.06 up to 16384 (fewer fp32 additions a sum).
 #include "ggq_cols.h"
 
 namespace ggq {
