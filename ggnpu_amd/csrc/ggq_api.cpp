@@ -101,6 +101,7 @@ struct ggq_ctx {
     Buffer aside;                // memory for captures, its first aside_used bytes in use
     size_t aside_used = 0, aside_total = 0;  // (total: outgrown allocations too)
     size_t lane_need = 0;        // the largest buffer an eager call asked for
+    size_t aside_refused = SIZE_MAX;  // memory for captures that could not be had
     Buffer io;  // staging of host A / C for the synchronous entry points
     Buffer logits;  // vocab projection output when the caller does not keep it
     Buffer attn;  // attention chunk partials
@@ -215,18 +216,25 @@ struct Want {
 bool grow_lane(ggq_ctx* c, Buffer& b, size_t bytes, const Want* wants, int n_wants) {
     c->lane_need = std::max(c->lane_need, bytes);
     // for eight captures in a row, two where that would be more than 256 MB
-    const size_t aside = aside_short(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
+    size_t aside = aside_short(c, c->lane_need, std::min<size_t>(8, std::max<size_t>(2, (size_t(256) << 20) / c->lane_need)));
+    if (aside >= c->aside_refused) aside = 0;  // not tried on each call anew
     const size_t lane = Want{&b, bytes}.grown();
-    size_t extra = aside;
-    for (int i = 0; i < n_wants; i++) extra += wants[i].grown();
-    if (!lane && !extra) return true;
-    char* p = (char*)alloc_beside_captures(lane + extra);
-    const bool all = p;
-    if (!p && lane && extra) p = (char*)alloc_beside_captures(lane);
+    size_t spare = 0;
+    for (int i = 0; i < n_wants; i++) spare += wants[i].grown();
+    if (!lane && !spare && !aside) return true;
+    char* p = (char*)alloc_beside_captures(lane + spare + aside);
+    if (!p && aside) {
+        c->aside_refused = aside;
+        aside = 0;
+        if (lane + spare) p = (char*)alloc_beside_captures(lane + spare);
+    }
+    if (!p && lane && spare) {
+        n_wants = 0;
+        p = (char*)alloc_beside_captures(lane);
+    }
     if (!p) return !lane;
     c->owned.push_back(p);
     if (lane) b = Buffer{p, lane};
-    if (!all) return true;
     p += lane;
     for (int i = 0; i < n_wants; i++)
         if (const size_t n = wants[i].grown()) {
