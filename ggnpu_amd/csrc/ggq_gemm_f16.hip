@@ -534,6 +534,28 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
             for (int e = 0; e < 8; e++) v[i][e] = in ? v[i][e] : 0.0f;
         }
     };
+    // the largest magnitude of each superblock in hand
+    float sx[RP / PP];
+    auto largest = [&] {
+#pragma unroll
+        for (int i0 = 0; i0 < RP; i0 += PP) {
+            float x = 0.0f;
+#pragma unroll
+            for (int j = 0; j < PP; j++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) x = fmaxf(x, fabsf(v[i0 + j][e]));
+            // the other pieces: in the sixteen lanes, then in the others
+            if constexpr (RW == 1) {
+                x = fmaxf(x, dpp<0x121>(x));
+                x = fmaxf(x, dpp<0x122>(x));
+            }
+            x = fmaxf(x, dpp<0x124>(x));
+            x = fmaxf(x, dpp<0x128>(x));
+            x = fmaxf(x, __shfl_xor(x, 16, 64));
+            if constexpr (RW == 4) x = fmaxf(x, __shfl_xor(x, 32, 64));
+            sx[i0 / PP] = x;
+        }
+    };
     int ex = 0;
     float inv = 0.0f;
     if constexpr (MODE == 2) {
@@ -542,13 +564,11 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
         float amax = 0.0f;
         for (int c = 0; c < np; c += chunk) {
             load(c);
+            largest();
 #pragma unroll
-            for (int i = 0; i < RP; i++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[i][e]));
+            for (int i = 0; i < RP / PP; i++) amax = fmaxf(amax, sx[i]);
         }
-#pragma unroll
-        for (int off = 32; off >= RW; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        if constexpr (RW == 1) amax = fmaxf(amax, __shfl_xor(amax, 32, 64));  // a wavefront's other superblock
         if (lane < RW) wmax[(tid >> 6) * RW + lane] = amax;
         __syncthreads();
         for (int o = 0; o < waves; o++) amax = fmaxf(amax, wmax[o * RW + tid % RW]);
@@ -560,7 +580,10 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
             inv = __fdiv_rn(1.0f, sc);
             if (tid < RW && m < a.M) a.rs[m] = sc;
         }
-        if (np > chunk) load(0);
+        if (np > chunk) {
+            load(0);
+            if constexpr (kSplit) largest();
+        }
     }
     for (int c = 0;;) {
 #pragma unroll
@@ -569,20 +592,7 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
             if (q0 >= np) break;
             int es = ex;
             if constexpr (kSplit) {
-                float smax = 0.0f;
-#pragma unroll
-                for (int j = 0; j < PP; j++)
-#pragma unroll
-                    for (int e = 0; e < 8; e++) smax = fmaxf(smax, fabsf(v[i0 + j][e]));
-                // the other pieces: in the sixteen lanes, then in the others
-                if constexpr (RW == 1) {
-                    smax = fmaxf(smax, dpp<0x121>(smax));
-                    smax = fmaxf(smax, dpp<0x122>(smax));
-                }
-                smax = fmaxf(smax, dpp<0x124>(smax));
-                smax = fmaxf(smax, dpp<0x128>(smax));
-                smax = fmaxf(smax, __shfl_xor(smax, 16, 64));
-                if constexpr (RW == 4) smax = fmaxf(smax, __shfl_xor(smax, 32, 64));
+                const float smax = sx[i0 / PP];
                 // its own from 2^4 below the row's on, at most 2^126 from it (a
                 // byte, an fp32 exponent)
                 if (smax > 0.0f && scale_exp(smax) - ex >= 4) es = min(scale_exp(smax), ex + 126);
@@ -617,6 +627,7 @@ __global__ __launch_bounds__(1024) void prep_kernel(PrepArgs a) {
         c += chunk;
         if (c >= np) break;
         load(c);
+        if constexpr (kSplit) largest();
     }
 }
 
